@@ -86,11 +86,12 @@ __device__ __forceinline__ const __attribute__((address_space(1))) T* gptr(const
 }
 
 // A lane's words of one k-slice: its K words with one non-temporal 64/96/128-bit buffer load
-// (+1 dword at K=5), and the word before them in the tile's circular bit string (the last word
-// of the previous lane of the tile, or the tile's last word for the first lane) with one more
-// dword load from the same cache lines. Buffer loads take the wave-uniform slice offset in a
-// scalar register and the per-lane offsets as constant vector offsets, so a step spends no
-// vector instructions on addresses.
+// (+1 dword at K=5). The word before them in the tile's circular bit string comes from the lane
+// that owns it (prev_word): a second load from the same cache lines cost more than the two
+// instructions of the exchange, since the vector memory path is as busy as the vector ALU here
+// (16 tokens at 4 bpw, MFMA tiles: 361 -> 327 us; 400 tokens at 3 bpw: 1850 -> 1719 us). Buffer
+// loads take the wave-uniform slice offset in a scalar register and the per-lane offsets as
+// constant vector offsets, so a step spends no vector instructions on addresses.
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -109,8 +110,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t weight_rsrc(const uint32_t* ba
 }
 
 template <int K>
-__device__ __forceinline__ void load_slice(LaneWords<K>& w, __amdgpu_buffer_rsrc_t rsrc, uint32_t soff,
-                                           uint32_t lane_off, uint32_t prev_off)
+__device__ __forceinline__ void load_slice(LaneWords<K>& w, __amdgpu_buffer_rsrc_t rsrc, uint32_t soff, uint32_t lane_off)
 {
     if constexpr (K == 2) {
         const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, lane_off, soff, BUF_NT));
@@ -124,7 +124,18 @@ __device__ __forceinline__ void load_slice(LaneWords<K>& w, __amdgpu_buffer_rsrc
 #pragma unroll
         for (int i = 4; i < K; ++i) w.b[i + 1] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, lane_off + 4 * i, soff, BUF_NT);
     }
-    w.b[0] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, prev_off, soff, BUF_NT);
+}
+
+// The word before a lane's own: the last word of the lane before it among the tile's 8 lanes,
+// circularly. A row of 16 lanes holds two tiles: rotated by one it gives every lane but each tile's
+// first its word, rotated by nine those two. (At half rates only the even lanes' windows reach into
+// the word before their own, and for them it is the previous lane's last word too.)
+template <int K>
+__device__ __forceinline__ uint32_t prev_word(const LaneWords<K>& w)
+{
+    const int r9 = __builtin_amdgcn_update_dpp(0, (int)w.b[K], 0x129, 0xf, 0xf, true);     // row_ror:9
+    const int r1 = __builtin_amdgcn_update_dpp(0, (int)w.b[K], 0x121, 0xf, 0xf, true);     // row_ror:1
+    return (uint32_t)((threadIdx.x & 7) == 0 ? r9 : r1);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -154,24 +165,18 @@ struct Rate {
     static constexpr int TW = HALF ? 4 * (2 * B + 1) : 8 * K; // words per tile
 };
 
-// Byte offsets of a lane's words within its tile (lane_off: the K words, prev_off: the word
-// before them in the tile's circular bit string) and, at half rates, the normalising shift.
+// Byte offset of a lane's K words within its tile group and, at half rates, the normalising shift.
 template <int K2>
-__device__ __forceinline__ void lane_offsets(int lane, uint32_t& lane_off, uint32_t& prev_off, uint32_t& sh)
+__device__ __forceinline__ void lane_offsets(int lane, uint32_t& lane_off, uint32_t& sh)
 {
     using R = Rate<K2>;
     const int q = lane & 7;
     sh = 0;
     if constexpr (!R::HALF) {
         lane_off = 4u * (uint32_t)((lane >> 3) * R::TW + q * R::K);
-        prev_off = 4u * (uint32_t)((lane >> 3) * R::TW + (q == 0 ? R::TW - 1 : q * R::K - 1));
     } else {
-        // words s0 .. s0+B+1 cover the lane's bits and the 16 before them; s0 = -1 (q = 0) wraps
-        // to the tile's last word, which is loaded on its own like the integer rates' b[0]
-        const int r0 = 16 * q * (2 * R::B + 1);
-        const int s0 = (r0 - 17 + 32) / 32 - 1;              // floor((r0 - 17) / 32)
-        lane_off = 4u * (uint32_t)((lane >> 3) * R::TW + s0 + 1);
-        prev_off = 4u * (uint32_t)((lane >> 3) * R::TW + (q == 0 ? R::TW - 1 : s0));
+        // the words from the one that holds the lane's first bit: 16 q (2 B + 1) bits into the tile
+        lane_off = 4u * (uint32_t)((lane >> 3) * R::TW + q * (2 * R::B + 1) / 2);
         sh = (q & 1) ? 0u : 16u;
     }
 }
@@ -179,10 +184,11 @@ __device__ __forceinline__ void lane_offsets(int lane, uint32_t& lane_off, uint3
 // The (1024 + bytesum) pairs of the lane's 32 positions of one k-slice:
 // wp[4u + 2c + kh] = column q + 8c, k = 8kh + 2u and 8kh + 2u + 1 (low half: even k).
 template <int K2>
-__device__ __forceinline__ void decode_slice(const LaneWords<Rate<K2>::K>& w, uint32_t sh, half2_t (&wp)[16])
+__device__ __forceinline__ void decode_slice(LaneWords<Rate<K2>::K>& w, uint32_t sh, half2_t (&wp)[16])
 {
     using R = Rate<K2>;
     constexpr int K = R::K, B = R::B;
+    w.b[0] = prev_word<K>(w);
     if constexpr (!R::HALF) {
 #define EVAMX_DEC_UNIT(U)                                \
         wp[4 * U + 0] = lane_hpair<K, 8 * U + 0>(w);     \
@@ -302,8 +308,8 @@ __device__ __forceinline__ void gemv_wave(const uint32_t* __restrict__ trellis, 
     const uint32_t slice = __builtin_amdgcn_readfirstlane(4u * (uint32_t)(nt_n * TW));
     const uint32_t cbase = __builtin_amdgcn_readfirstlane(4u * (uint32_t)(cg * 8 * TW));
     const __amdgpu_buffer_rsrc_t rsrc = weight_rsrc(trellis);
-    uint32_t lane_off, prev_off, sh;
-    lane_offsets<K2>(lane, lane_off, prev_off, sh);
+    uint32_t lane_off, sh;
+    lane_offsets<K2>(lane, lane_off, sh);
 
     // Prefetch ring: the row PF slices ahead, clamped to the wave's last row so that the steady
     // state needs no branch and never reads outside the matrix (the clamped reloads hit cache).
@@ -311,7 +317,7 @@ __device__ __forceinline__ void gemv_wave(const uint32_t* __restrict__ trellis, 
     LaneWords<K> ring[PF];
     const int last = kt1 - 1;
 #pragma unroll
-    for (int d = 0; d < PF; ++d) load_slice<K>(ring[d], rsrc, cbase + (uint32_t)min(kt0 + d, last) * slice, lane_off, prev_off);
+    for (int d = 0; d < PF; ++d) load_slice<K>(ring[d], rsrc, cbase + (uint32_t)min(kt0 + d, last) * slice, lane_off);
     // keep the prologue's work (and its waits for its own loads) after the ring is issued
     if constexpr (Pro::kWork) __builtin_amdgcn_sched_barrier(0);
     prologue.finish();
@@ -335,7 +341,7 @@ __device__ __forceinline__ void gemv_wave(const uint32_t* __restrict__ trellis, 
         if constexpr (XPF) load_x(xn, min(kt + 1, last));
         half2_t wp[16];
         decode_slice<K2>(w, sh, wp);
-        load_slice<K>(w, rsrc, cbase + (uint32_t)min(kt + PF, last) * slice, lane_off, prev_off);
+        load_slice<K>(w, rsrc, cbase + (uint32_t)min(kt + PF, last) * slice, lane_off);
 #pragma unroll
         for (int m = 0; m < TM; ++m) {
             if (m < tm) {
@@ -451,14 +457,14 @@ __device__ __forceinline__ void gemv_wave_m4(const uint32_t* __restrict__ trelli
     const uint32_t slice = __builtin_amdgcn_readfirstlane(4u * (uint32_t)(nt_n * TW));
     const uint32_t cbase = __builtin_amdgcn_readfirstlane(4u * (uint32_t)(cg * 8 * TW));
     const __amdgpu_buffer_rsrc_t rsrc = weight_rsrc(trellis);
-    uint32_t lane_off, prev_off, sh;
-    lane_offsets<K2>(lane, lane_off, prev_off, sh);
+    uint32_t lane_off, sh;
+    lane_offsets<K2>(lane, lane_off, sh);
 
     prologue.issue();
     LaneWords<K> ring[PF];
     const int last = kt1 - 1;
 #pragma unroll
-    for (int d = 0; d < PF; ++d) load_slice<K>(ring[d], rsrc, cbase + (uint32_t)min(kt0 + d, last) * slice, lane_off, prev_off);
+    for (int d = 0; d < PF; ++d) load_slice<K>(ring[d], rsrc, cbase + (uint32_t)min(kt0 + d, last) * slice, lane_off);
     if constexpr (Pro::kWork) __builtin_amdgcn_sched_barrier(0);
     prologue.finish();
 
@@ -474,7 +480,7 @@ __device__ __forceinline__ void gemv_wave_m4(const uint32_t* __restrict__ trelli
             for (int g = 0; g < NA; ++g) xs.load(g, kt, xa[g]);
             half2_t wp[16];
             decode_slice<K2>(w, sh, wp);
-            load_slice<K>(w, rsrc, cbase + (uint32_t)min(kt + PF, last) * slice, lane_off, prev_off);
+            load_slice<K>(w, rsrc, cbase + (uint32_t)min(kt + PF, last) * slice, lane_off);
 #pragma unroll
             for (int kg = 0; kg < 4; ++kg)
 #pragma unroll

@@ -321,18 +321,17 @@ __global__ __launch_bounds__(256) void lin_rotate_kernel(LinParams p)
 // (codebook map with its rows' activation sums); the partials meet in LDS, added in wave order,
 // and every wave then runs the output epilogue of some of the tile's rows.
 template <int K2, int MB>
-__device__ __forceinline__ void lin_mfma_tile(const LinParams& p, int r0, int rows, int cg, uint32_t* stage,
-                                              float (*red)[132])
+__device__ __forceinline__ void lin_mfma_tile(const LinParams& p, int r0, int rows, int cg, float (*red)[132])
 {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int m16 = lane & 15, g = lane >> 4;
+    const int g = lane >> 4;
     const int nch = p.in / 128;
     const GlobalRows src{p.xr + (size_t)r0 * p.in, (size_t)p.in, p.xsum + (size_t)r0 * nch, nch};
     float pv[MB][8][4];
     if (wave < p.ks) {
         const int c0 = nch * wave / p.ks, c1 = nch * (wave + 1) / p.ks;
         f32x4_t acc[MB][8];
-        mfma_accumulate<K2, MB, false>(p.trellis, p.out / 16, cg, 8 * c0, 8 * c1, src, k_iota64, rows, stage, acc);
+        mfma_accumulate<K2, MB, false>(p.trellis, p.out / 16, cg, 8 * c0, 8 * c1, src, k_iota64, rows, acc);
         float xs[MB][4];
         mfma_row_sums<MB>(src, k_iota64, rows, 8 * c0, 8 * (c1 - c0), xs);
 #pragma unroll
@@ -353,7 +352,7 @@ __device__ __forceinline__ void lin_mfma_tile(const LinParams& p, int r0, int ro
                     if (row < rows) {
 #pragma unroll
                         for (int nb = 0; nb < 8; ++nb) {
-                            float* d = &red[row][16 * nb + m16];
+                            float* d = &red[row][mfma_col(lane, nb)];
                             *d = w == 0 ? pv[mb][nb][r] : *d + pv[mb][nb][r];
                         }
                     }
@@ -376,33 +375,30 @@ __device__ __forceinline__ void lin_mfma_tile(const LinParams& p, int r0, int ro
 }
 
 template <int K2>
-__device__ __forceinline__ void lin_mfma_rows(const LinParams& p, int r0, int rows, int cg, uint32_t* stage,
-                                              float (*red)[132])
+__device__ __forceinline__ void lin_mfma_rows(const LinParams& p, int r0, int rows, int cg, float (*red)[132])
 {
     switch (__builtin_amdgcn_readfirstlane((rows + 15) >> 4)) {
-        case 1: lin_mfma_tile<K2, 1>(p, r0, rows, cg, stage, red); break;
-        case 2: lin_mfma_tile<K2, 2>(p, r0, rows, cg, stage, red); break;
-        case 3: lin_mfma_tile<K2, 3>(p, r0, rows, cg, stage, red); break;
-        default: lin_mfma_tile<K2, 4>(p, r0, rows, cg, stage, red); break;
+        case 1: lin_mfma_tile<K2, 1>(p, r0, rows, cg, red); break;
+        case 2: lin_mfma_tile<K2, 2>(p, r0, rows, cg, red); break;
+        case 3: lin_mfma_tile<K2, 3>(p, r0, rows, cg, red); break;
+        default: lin_mfma_tile<K2, 4>(p, r0, rows, cg, red); break;
     }
 }
 
 __global__ __launch_bounds__(64 * LM_WAVES) void lin_mfma_kernel(LinParams p)
 {
-    __shared__ uint32_t stage[LM_WAVES][MF_LDS_WORDS];
     __shared__ float red[64][132];      // padded rows: the partial stores hit 64 distinct banks
     const int ncg = p.out / 128;
     const int tile = blockIdx.x / ncg, cg = blockIdx.x % ncg;
     const int r0 = 64 * tile, rows = p.rows - r0 < 64 ? p.rows - r0 : 64;
-    uint32_t* st = stage[threadIdx.x >> 6];
     switch (p.k2) {
-        case 3: lin_mfma_rows<3>(p, r0, rows, cg, st, red); break;
-        case 4: lin_mfma_rows<4>(p, r0, rows, cg, st, red); break;
-        case 5: lin_mfma_rows<5>(p, r0, rows, cg, st, red); break;
-        case 6: lin_mfma_rows<6>(p, r0, rows, cg, st, red); break;
-        case 7: lin_mfma_rows<7>(p, r0, rows, cg, st, red); break;
-        case 8: lin_mfma_rows<8>(p, r0, rows, cg, st, red); break;
-        case 10: lin_mfma_rows<10>(p, r0, rows, cg, st, red); break;
+        case 3: lin_mfma_rows<3>(p, r0, rows, cg, red); break;
+        case 4: lin_mfma_rows<4>(p, r0, rows, cg, red); break;
+        case 5: lin_mfma_rows<5>(p, r0, rows, cg, red); break;
+        case 6: lin_mfma_rows<6>(p, r0, rows, cg, red); break;
+        case 7: lin_mfma_rows<7>(p, r0, rows, cg, red); break;
+        case 8: lin_mfma_rows<8>(p, r0, rows, cg, red); break;
+        case 10: lin_mfma_rows<10>(p, r0, rows, cg, red); break;
         default: break;                 // the rate is validated on the host
     }
 }

@@ -1,23 +1,18 @@
-// Prefill-shaped expert GEMMs on gfx950: trellis decode into LDS feeding fp16 MFMA.
+// Prefill-shaped expert GEMMs on gfx950: trellis decode feeding fp16 MFMA in registers.
 //
 // Replaces the reference's grouped expert matmuls for large batches (the coop kernels'
 // gemv_tile, exl3_moe_coop_kernel.cuh:340-544, run once per <= 8-row run). Here a work item is
 // (tile of <= 64 grouped rows of one expert, 128 output columns, projection), one wave each,
-// over the full k range, so every weight is decoded once per 64 rows instead of once per 8:
+// over the full k range, so every weight is decoded once per 64 rows instead of once per 8 (the
+// core is mfma_accumulate, evamx_mfma.hpp). 4 x 8 accumulators (64 rows x 128 columns, fp32) take
+// sum_k x_k h_k, and the epilogue applies the codebook map per column with the rows' activation
+// sums, as the decode GEMV does, writing the same fp32 partials (one k-split).
 //
-//   - the wave streams its 8 trellis tiles per k-slice exactly like the decode GEMV (lane
-//     8*i + q owns tile i's columns q, q + 8) and decodes two k-slices into the (1024 +
-//     bytesum) fp16 values of the affine codebook map (w = 0x1eee * h + 0xc931);
-//   - it restages them through a wave-private 8 KiB LDS region into the B operands of
-//     v_mfma_f32_16x16x32_f16 (lane n + 16 g holds column n, k = 8g .. 8g+7), one per 16-column
-//     tile, and reads the rotated activations of its rows as the A operands (lane m + 16 g
-//     holds row m, the same k) straight from global memory;
-//   - 4 x 8 accumulators (64 rows x 128 columns, fp32) take sum_k x_k h_k, and the epilogue
-//     applies the codebook map per column with the rows' activation sums, as the decode GEMV
-//     does, writing the same fp32 partials (one k-split).
-//
-// The LDS exchange stays within a wave (a wave's LDS instructions execute in order), so the
-// waves of a workgroup never synchronise.
+// What bounds it: the decode's vector instructions (3.4 to 3.9 per weight) and, next to them, the
+// vector memory path. Taking the decoded slices as MFMA operands where they are (they went through
+// LDS before) and the previous words from the neighbour lane (they were a second load) gave, start
+// against now on one box: 16 tokens at 4 bpw 412 -> 368 us a layer, 512 tokens at mixed rates
+// 1630 -> 1446 us, 3001 tokens 6739 -> 5839 us.
 //
 // Calls of more than 16 tokens run two kernels per stage: the tiles of at most 16 rows in the
 // 16-row kernel (a quarter of the accumulators, 4 waves per SIMD) on the calling thread's side
@@ -39,20 +34,20 @@ constexpr int MF_WAVES = 4;                     // waves per workgroup
 template <int K2, int MBMAX>
 __device__ __forceinline__ void mfma_item_rows(const uint32_t* trellis, int nt_n, int cg, int kt0, int kt1,
                                                const GlobalRows& src, const int* slot_of, int rows, float* part,
-                                               size_t part_stride, uint32_t* lds)
+                                               size_t part_stride)
 {
     // both kernels run their items with progress priorities: the 16-row kernel's equal items,
     // and the 64-row kernel's items of 1-4 row blocks since they share the GPU with the 16-row
     // kernel on another stream (512 tokens: gate/up 1319-1331 -> 1268-1287 us)
     if constexpr (MBMAX == 1) {
-        mfma_item<K2, 1, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride, lds);
+        mfma_item<K2, 1, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride);
     } else {
         const int mb = __builtin_amdgcn_readfirstlane((rows + 15) >> 4);
         switch (mb) {
-            case 1: mfma_item<K2, 1, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride, lds); break;
-            case 2: mfma_item<K2, 2, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride, lds); break;
-            case 3: mfma_item<K2, 3, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride, lds); break;
-            default: mfma_item<K2, 4, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride, lds); break;
+            case 1: mfma_item<K2, 1, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+            case 2: mfma_item<K2, 2, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+            case 3: mfma_item<K2, 3, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+            default: mfma_item<K2, 4, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
         }
     }
 }
@@ -75,7 +70,7 @@ __device__ __forceinline__ int xcd_item_block(int b, int nb)
 // (a quarter of the accumulators, 4 waves per SIMD) runs the tiles of at most 16 rows, the
 // MBMAX 4 kernel the larger ones; the split count is the same for both (from all the tiles).
 template <int MBMAX, int which>
-__device__ __forceinline__ void mfma_stage(const MoeParams& p, uint32_t (&lds)[MF_WAVES][MF_LDS_WORDS])
+__device__ __forceinline__ void mfma_stage(const MoeParams& p)
 {
     const int wave = threadIdx.x >> 6;
     const int n_all = __builtin_amdgcn_readfirstlane(p.meta[0]);
@@ -135,15 +130,14 @@ __device__ __forceinline__ void mfma_stage(const MoeParams& p, uint32_t (&lds)[M
         nt_n = p.H / 16;
     }
     const int kt0 = 8 * (nch * ks / S), kt1 = 8 * (nch * (ks + 1) / S);
-    uint32_t* wl = lds[wave];
     switch (k2) {
-        case 3: mfma_item_rows<3, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride, wl); break;
-        case 4: mfma_item_rows<4, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride, wl); break;
-        case 5: mfma_item_rows<5, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride, wl); break;
-        case 6: mfma_item_rows<6, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride, wl); break;
-        case 7: mfma_item_rows<7, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride, wl); break;
-        case 8: mfma_item_rows<8, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride, wl); break;
-        case 10: mfma_item_rows<10, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride, wl); break;
+        case 3: mfma_item_rows<3, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+        case 4: mfma_item_rows<4, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+        case 5: mfma_item_rows<5, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+        case 6: mfma_item_rows<6, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+        case 7: mfma_item_rows<7, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+        case 8: mfma_item_rows<8, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+        case 10: mfma_item_rows<10, MBMAX>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
         default: {
             // unsupported rate (flagged by the grouping): zero partials, so no output reads stale data
             const int lane = threadIdx.x & 63;
@@ -161,15 +155,13 @@ __device__ __forceinline__ void mfma_stage(const MoeParams& p, uint32_t (&lds)[M
 template <int MBMAX>
 __global__ __launch_bounds__(64 * MF_WAVES) __attribute__((amdgpu_waves_per_eu(MBMAX == 1 ? 3 : 2))) void moe_gate_up_mfma_kernel(MoeParams p)
 {
-    __shared__ uint32_t lds[MF_WAVES][MF_LDS_WORDS];
-    mfma_stage<MBMAX, 0>(p, lds);
+    mfma_stage<MBMAX, 0>(p);
 }
 
 template <int MBMAX>
 __global__ __launch_bounds__(64 * MF_WAVES) __attribute__((amdgpu_waves_per_eu(MBMAX == 1 ? 3 : 2))) void moe_down_mfma_kernel(MoeParams p)
 {
-    __shared__ uint32_t lds[MF_WAVES][MF_LDS_WORDS];
-    mfma_stage<MBMAX, 1>(p, lds);
+    mfma_stage<MBMAX, 1>(p);
 }
 
 // Side stream of the calling thread on the current device, with its fork and join events, for
