@@ -76,12 +76,10 @@ __device__ __forceinline__ uint16_t bf16_bits(float f)
 
 // ---------------------------------------------------------------------------------------------
 // Router front: logits[r][e] = sum_k float(x[r][k]) * gate_w[e][k] in fp32 (Block.route's
-// x.float() @ gate_w.T, model.py:404-409). One wave per (expert, group of GATE_ROWS rows): lane l
-// takes k = 4l + 256j (one float4 of the weight row per step, reused by the group's rows) with a
-// sequential fma chain, and the lanes' partials meet in a fixed butterfly, so a row's logits
-// depend on that row alone whatever the batch (the per-row stable_linear of model.py:158-165).
-
-constexpr int GATE_ROWS = 8;
+// x.float() @ gate_w.T, model.py:404-409). One wave per (group of rows, group of experts): lane l
+// takes k = 4l + 256j with a sequential fma chain for each (row, expert), and the lanes' partials
+// meet in a fixed butterfly, so a row's logits depend on that row alone whatever the batch or the
+// groups (the per-row stable_linear of model.py:158-165).
 
 // x as the fp16 value the reference routes and runs the experts on: Block.experts casts the
 // activations to fp16 first (model.py:455), so a bf16 x is rounded to fp16 (values beyond the

@@ -196,3 +196,23 @@ def test_router_logits_round_bf16_x_to_fp16(dev):
     with pytest.raises(AssertionError):                  # the unrounded values miss the bound
         _check_logits(z[1:2], x[1:2], gate_w)
     assert np.all(np.isinf(z[2])) and np.array_equal(np.sign(z[2]), np.sign(gate_w[:, 100]))
+
+
+@pytest.mark.parametrize("rows,E,H", [(1, 3, 132), (1, 257, 260), (2, 5, 512), (9, 64, 1028), (31, 255, 384), (33, 192, 644),
+                                      (96, 256, 384), (97, 257, 516), (203, 129, 2052)])
+@pytest.mark.parametrize("shift", [0, 1, 2])
+def test_router_logits_tiles(dev, rows, E, H, shift):
+    """Every tile of the gate kernel at its edges (rows and experts short of a tile, fewer row groups
+    than a workgroup's waves, widths short of a wave's stride), with rows 8-, 2- and 4-byte aligned:
+    within the accumulation bound, and bit-identical to the rows' one-row calls on aligned copies."""
+    ops = _ops()
+    rng = np.random.default_rng(rows * 1000 + E + shift)
+    x = synth.activations_bf16(rng, rows, H)
+    gate_w = to_dev(_gate(rng, E, H), dev)
+    wide = torch.zeros(rows, H + 4 + shift, dtype=torch.float16, device=dev)
+    wide[:, shift:shift + H] = to_dev(x, dev)
+    xt = wide[:, shift:shift + H]
+    z = ops.router_logits(xt, gate_w)
+    _check_logits(z.cpu().numpy(), xt.float().cpu().numpy(), gate_w.cpu().numpy())
+    for r in {0, rows // 2, rows - 1}:
+        assert torch.equal(ops.router_logits(xt[r:r + 1].contiguous(), gate_w)[0], z[r])
