@@ -38,6 +38,38 @@ __device__ __forceinline__ int mfma_col(int lane, int nb)
     return 32 * (nb >> 1) + 16 * ((lane >> 3) & 1) + 8 * (nb & 1) + (lane & 7);
 }
 
+// had128_lane for a row's 128 values in the accumulator layout, value nb at column mfma_col(lane, nb):
+// bits 0-2 and 4 of the column are lane bits 0-3, bits 3, 5 and 6 are bits of nb. Same stages in the
+// same order, so the results are bit-identical.
+__device__ __forceinline__ void had128_acc(float (&v)[8], int lane)
+{
+#pragma unroll
+    for (int nb = 0; nb < 8; ++nb) v[nb] = bfly_x<4>(bfly_x<2>(bfly_x<1>(v[nb], lane), lane), lane);
+#pragma unroll
+    for (int nb = 0; nb < 8; nb += 2) {
+        const float a = v[nb], c = v[nb + 1];
+        v[nb] = a + c;
+        v[nb + 1] = a - c;
+    }
+#pragma unroll
+    for (int nb = 0; nb < 8; ++nb) v[nb] = bfly_x<8>(v[nb], lane);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int nb = (i & 1) + 4 * (i >> 1);               // nb bit 1: column bit 5
+        const float a = v[nb], c = v[nb + 2];
+        v[nb] = a + c;
+        v[nb + 2] = a - c;
+    }
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {                         // nb bit 2: column bit 6
+        const float a = v[nb], c = v[nb + 4];
+        v[nb] = a + c;
+        v[nb + 4] = a - c;
+    }
+#pragma unroll
+    for (int nb = 0; nb < 8; ++nb) v[nb] *= R_SCALE;
+}
+
 // Accumulators of one work item: rows [0, rows) (slots slot_of[0..rows)) of activations src
 // (fp16 [slot][K] with 128-chunk sums) times the (1024 + bytesum) values of tiles 8*cg .. 8*cg+7
 // of a projection over the k-slices [kt0, kt1) (whole 128-chunks): acc[mb][nb][r] = sum_k x_k h_k
@@ -116,6 +148,76 @@ __device__ __forceinline__ void mfma_accumulate(const uint32_t* __restrict__ tre
             for (int h = 0; h < 2; ++h) a[mb][h] = an[mb][h];
     }
     if constexpr (PRIO) progress_priority(1, 1);
+}
+
+// Activations laid out as A operands: a block of 16 rows is, for each k64 step t and k half h, the 64
+// lanes' 16 bytes in lane order (row m16, k = 64 t + 16 g + 8 h ..), 1 KiB a load. Read from plain rows
+// instead, the lanes of a load lie in 16 rows and each takes an address cycle of its own, four times the
+// load's data cycles (64 rows, 7168 x 2048: 115 us a call, all of it these loads). Byte offset of the
+// block with row 16 b, K columns.
+__host__ __device__ __forceinline__ size_t a_operand_offset(int b, int K) { return (size_t)b * 16 * K * 2; }
+
+// The same products for one pair of tiles (32 columns) over `chunks` 128-chunks of k: acc[mb][c][r] +=
+// for row 16 mb + 4 g + r and column mfma_col(lane, c) of the pair, rows at arow[mb] (the lane's k-slice
+// group g). pair: the pair's index among the projection's column tiles. Weights three steps of 64 k in
+// flight, activations two. end(i) runs after chunk i.
+template <int K2, int MB, typename End>
+__device__ __forceinline__ void mfma_pair(const uint32_t* __restrict__ trellis, int nt_n, int pair, int kt0, int chunks,
+                                          const __attribute__((address_space(1))) u32x4_t* const (&arow)[MB], f32x4_t (&acc)[MB][2],
+                                          End&& end)
+{
+    using R = Rate<K2>;
+    constexpr int K = R::K;
+    constexpr int TW = R::TW;
+    const int lane = threadIdx.x & 63;
+    const int last = 2 * chunks - 1;
+    const uint32_t slice = __builtin_amdgcn_readfirstlane(4u * (uint32_t)(nt_n * TW));
+    const uint32_t cbase = __builtin_amdgcn_readfirstlane(4u * (uint32_t)(2 * pair * TW) + (uint32_t)kt0 * slice);
+    const __amdgpu_buffer_rsrc_t rsrc = weight_rsrc(trellis);
+    uint32_t lane_off, sh;
+    lane_offsets<K2>(lane & 15, lane_off, sh);
+    lane_off += (uint32_t)(lane >> 4) * slice;
+    LaneWords<K> ring[3];
+    u32x4_t a[3][MB][2];
+    auto load_w = [&](LaneWords<K>& w, int t) { load_slice<K>(w, rsrc, cbase + (uint32_t)(4 * min(t, last)) * slice, lane_off); };
+    auto load_a = [&](u32x4_t (&d)[MB][2], int t) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) d[mb][h] = arow[mb][128 * min(t, last) + 64 * h];
+    };
+    auto step = [&](int t, LaneWords<K>& w, const u32x4_t (&x)[MB][2], u32x4_t (&y)[MB][2]) {
+        load_a(y, t + 2);
+        half2_t wp[16];
+        decode_slice<K2>(w, sh, wp);
+        load_w(w, t + 3);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const half8_t b = mfma_b(wp, c, h);
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+                    acc[mb][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, x[mb][h]), b, acc[mb][c], 0, 0, 0);
+            }
+    };
+#pragma unroll
+    for (int d = 0; d < 3; ++d) load_w(ring[d], d);
+    load_a(a[0], 0);
+    load_a(a[1], 1);
+    for (int i = 0; i < chunks; i += 3) {
+        step(2 * i, ring[0], a[0], a[2]);
+        step(2 * i + 1, ring[1], a[1], a[0]);
+        end(i);
+        if (i + 1 >= chunks) break;
+        step(2 * i + 2, ring[2], a[2], a[1]);
+        step(2 * i + 3, ring[0], a[0], a[2]);
+        end(i + 1);
+        if (i + 2 >= chunks) break;
+        step(2 * i + 4, ring[1], a[1], a[0]);
+        step(2 * i + 5, ring[2], a[2], a[1]);
+        end(i + 2);
+    }
 }
 
 // Activation sums over the k-slices [kt0, kt0 + nk) of the rows whose accumulators a lane holds:

@@ -9,12 +9,14 @@
 // output epilogue (the partials summed in fixed split order, fp16 C, Hadamard, fp16 svh product).
 // 3 to 16 rows, three launches: the input rotation, the same GEMV on the rotated rows, and the
 // same epilogue in a launch of its own.
-// More rows, two launches: the input rotation, then the MFMA path, one workgroup per (64-row
-// tile, 128 output columns) whose waves take fixed k-ranges, meet in LDS (summed in wave
-// order) and run the output epilogue. In both paths a row's arithmetic depends on in/out only,
-// not on how many rows share the call.
+// More rows: the input rotation, written as MFMA operands, then one of three MFMA kernels by size
+// (linear_kind): 256-row workgroups that share each decoded weight (lin_wide_kernel), 64-row
+// workgroups over the whole k range, or over one k-range each with the output epilogue in a launch
+// of its own. All add the same k-ranges' sums in the same order. In both paths (up to
+// LIN_GEMV_ROWS rows, and beyond) a row's arithmetic depends on in/out only, not on how many rows
+// share the call.
 #include "evamx_internal.hpp"
-#include "evamx_mfma.hpp"
+#include "evamx_wide.hpp"
 
 namespace evamx {
 
@@ -294,7 +296,7 @@ void launch_gemv_rate(const LinParams& p, hipStream_t stream)
 // ---------------------------------------------------------------------------------------------
 // More than LIN_GEMV_ROWS rows (and the rotation of 3 to LIN_GEMV_ROWS rows).
 
-constexpr int LM_WAVES = 8;           // waves (k-ranges) per workgroup of the MFMA path
+constexpr int LIN_RANGES = 8;         // k-ranges whose sums are added in order
 
 // fp16(H128(fp16(x * suh))) of every (row, 128-chunk) with the chunk's sum: one wave each.
 __global__ __launch_bounds__(256) void lin_rotate_kernel(LinParams p)
@@ -316,99 +318,302 @@ __global__ __launch_bounds__(256) void lin_rotate_kernel(LinParams p)
     if (lane == 0) p.xsum[(size_t)r * nch + c] = sum;
 }
 
-// One workgroup per (tile of up to 64 rows, 128 output columns); wave w < p.ks streams the
-// 128-chunks [nch w / ks, nch (w + 1) / ks) into MFMA accumulators and forms its partials
-// (codebook map with its rows' activation sums); the partials meet in LDS, added in wave order,
-// and every wave then runs the output epilogue of some of the tile's rows.
-template <int K2, int MB>
-__device__ __forceinline__ void lin_mfma_tile(const LinParams& p, int r0, int rows, int cg, float (*red)[132])
+// The same rotations for calls of more than LIN_GEMV_ROWS rows, written as A operands
+// (a_operand_offset): one workgroup per (16 rows, 128-chunk), each wave four rows, which meet in LDS and
+// leave as the chunk's 4 KiB. Rows past the call's are zero.
+__global__ __launch_bounds__(256) void lin_rotate16_kernel(LinParams p)
 {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __shared__ half_t sh[16][136];                       // padded rows
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nch = p.in / 128;
+    const int b = blockIdx.x / nch, c = blockIdx.x % nch;
+    const half2_t su = __builtin_bit_cast(half2_t, ((const uint32_t*)(p.suh + c * 128))[lane]);
+    uint32_t xw[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        xw[i] = ((const uint32_t*)(p.x + (size_t)min(16 * b + 4 * wave + i, p.rows - 1) * p.in + c * 128))[lane];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = 16 * b + 4 * wave + i;
+        const half2_t xx = __builtin_bit_cast(half2_t, xw[i]);
+        float v0 = h2f(f2h(h2f(xx.x) * h2f(su.x)));      // fp16 product
+        float v1 = h2f(f2h(h2f(xx.y) * h2f(su.y)));
+        had128_pair(v0, v1, lane);
+        const half2_t o = {f2h(v0), f2h(v1)};
+        *(uint32_t*)&sh[4 * wave + i][2 * lane] = r < p.rows ? __builtin_bit_cast(uint32_t, o) : 0u;
+        const float sum = wave_sum(h2f(o.x) + h2f(o.y));
+        if (lane == 0 && r < p.rows) p.xsum[(size_t)r * nch + c] = sum;
+    }
+    __syncthreads();
+    // thread -> operand (k64 step wave >> 1, half wave & 1), lane
+    const int m16 = lane & 15, g = lane >> 4;
+    const u32x4_t v = *(const u32x4_t*)&sh[m16][64 * (wave >> 1) + 16 * g + 8 * (wave & 1)];
+    ((u32x4_t*)((char*)p.xr + a_operand_offset(b, p.in)))[(4 * c + wave) * 64 + lane] = v;
+}
+
+// Activation sum of a row: its 128-chunk sums, lane l those of chunks l, l + 64, ..., then the wave's
+// butterfly. Every kernel for more than LIN_GEMV_ROWS rows takes it (and the k-ranges' sums in range
+// order), so a row's result does not depend on which of them its call runs.
+__device__ __forceinline__ float lin_row_total(const LinParams& p, int row)
+{
+    const int nch = p.in / 128;
+    return wave_sum(strided_sum<2>(p.xsum + (size_t)row * nch, threadIdx.x & 63, nch, 64));
+}
+
+// Output epilogue of a row's 128 accumulated columns (the lane's two): codebook map, C in fp16, Hadamard,
+// fp16 svh product.
+__device__ __forceinline__ void lin_store_row(const LinParams& p, int row, int cg, float v0, float v1, float xs, const float (&sv)[2])
+{
+    const int lane = threadIdx.x & 63;
+    v0 = h2f(f2h(mul1_affine(v0, xs)));
+    v1 = h2f(f2h(mul1_affine(v1, xs)));
+    had128_lane(v0, v1, lane);
+    half_t* y = p.y + (size_t)row * p.out + cg * 128 + lane_col(lane, 0);
+    y[0] = f2h(h2f(f2h(v0)) * sv[0]);
+    y[8] = f2h(h2f(f2h(v1)) * sv[1]);
+}
+
+// Calls of more than LIN_GEMV_ROWS rows with too few wide tiles to fill the device: one workgroup per
+// tile of up to 64 rows and 128 output columns, wave j taking the pair j of the group's tiles, whose
+// decoded weights stay in its registers. The waves read the same activations, which the CU's cache
+// serves. SPLIT: a workgroup takes one k-range and stores its accumulators as partials
+// (lin_mid_epilogue_kernel adds the ranges); otherwise all of them, added in order, and the output
+// epilogue meets in LDS.
+constexpr int LM_ROWS = 64;
+constexpr int LM_WAVES = 4;
+
+template <int K2, int MB, bool SPLIT>
+__device__ __forceinline__ void lin_mid_tile(const LinParams& p, int r0, int rows, int cg, int range, float (*red)[132])
+{
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int g = lane >> 4;
     const int nch = p.in / 128;
-    const GlobalRows src{p.xr + (size_t)r0 * p.in, (size_t)p.in, p.xsum + (size_t)r0 * nch, nch};
-    float pv[MB][8][4];
-    if (wave < p.ks) {
-        const int c0 = nch * wave / p.ks, c1 = nch * (wave + 1) / p.ks;
-        f32x4_t acc[MB][8];
-        mfma_accumulate<K2, MB, false>(p.trellis, p.out / 16, cg, 8 * c0, 8 * c1, src, k_iota64, rows, acc);
-        float xs[MB][4];
-        mfma_row_sums<MB>(src, k_iota64, rows, 8 * c0, 8 * (c1 - c0), xs);
+    const int c0 = SPLIT ? nch * range / p.ks : 0, c1 = SPLIT ? nch * (range + 1) / p.ks : nch;
+    const __attribute__((address_space(1))) u32x4_t* arow[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+        arow[mb] = (const __attribute__((address_space(1))) u32x4_t*)((const char*)p.xr + a_operand_offset(r0 / 16 + mb, p.in)) + 256 * c0 + lane;
+    f32x4_t acc[MB][2], tot[MB][2];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) acc[mb][c] = tot[mb][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    int n = 0, stop = nch / p.ks;                                // the chunk after the range's last
+    mfma_pair<K2, MB>(p.trellis, p.out / 16, 4 * cg + wave, 8 * c0, c1 - c0, arow, acc, [&](int i) {
+        if (SPLIT || i + 1 != stop) return;
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-            for (int nb = 0; nb < 8; ++nb)
+            for (int c = 0; c < 2; ++c) {
+                tot[mb][c] += acc[mb][c];
+                acc[mb][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        ++n;
+        stop = nch * (n + 1) / p.ks;
+    });
+    float* part = SPLIT ? p.part + ((size_t)range * p.rows + r0) * p.out + 128 * cg + 32 * wave : nullptr;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) pv[mb][nb][r] = mul1_affine(acc[mb][nb][r], xs[mb][r]);
-    }
-    for (int w = 0; w < p.ks; ++w) {
-        __syncthreads();
-        if (wave == w) {
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
+        for (int r = 0; r < 4; ++r) {
+            const int row = 16 * mb + 4 * g + r;
+            if (row < rows) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = 16 * mb + 4 * g + r;
-                    if (row < rows) {
-#pragma unroll
-                        for (int nb = 0; nb < 8; ++nb) {
-                            float* d = &red[row][mfma_col(lane, nb)];
-                            *d = w == 0 ? pv[mb][nb][r] : *d + pv[mb][nb][r];
-                        }
-                    }
+                for (int c = 0; c < 2; ++c) {
+                    if constexpr (SPLIT) part[(size_t)row * p.out + mfma_col(lane, c)] = acc[mb][c][r];
+                    else red[row][32 * wave + mfma_col(lane, c)] = tot[mb][c][r];
                 }
+            }
+        }
+    if constexpr (!SPLIT) {
+        __syncthreads();
+        float sv[2];
+        lin_load_sv(p, cg, sv);
+        for (int row = wave; row < rows; row += LM_WAVES) {
+            const float xs = lin_row_total(p, r0 + row);
+            lin_store_row(p, r0 + row, cg, red[row][lane_col(lane, 0)], red[row][lane_col(lane, 1)], xs, sv);
         }
     }
-    __syncthreads();
-    float sv[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) sv[h] = h2f(p.svh[cg * 128 + lane_col(lane, h)]);
-    for (int row = wave; row < rows; row += LM_WAVES) {
-        float v[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) v[h] = h2f(f2h(red[row][lane_col(lane, h)]));     // C in fp16
-        had128_lane(v[0], v[1], lane);
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-            p.y[(size_t)(r0 + row) * p.out + cg * 128 + lane_col(lane, h)] = f2h(h2f(f2h(v[h])) * sv[h]);
+}
+
+template <int K2, bool SPLIT>
+__global__ __launch_bounds__(64 * LM_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void lin_mid_kernel(LinParams p)
+{
+    __shared__ float red[SPLIT ? 1 : LM_ROWS][132];              // padded rows
+    // ranges fastest: the workgroups of a tile and column group run side by side
+    const int nr = SPLIT ? p.ks : 1;
+    const int range = blockIdx.x % nr, rest = blockIdx.x / nr, ncg = p.out / 128;
+    const int r0 = rest / ncg * LM_ROWS, cg = rest % ncg;
+    const int rows = min(LM_ROWS, p.rows - r0);
+    switch (__builtin_amdgcn_readfirstlane((rows + 15) >> 4)) {
+        case 1: lin_mid_tile<K2, 1, SPLIT>(p, r0, rows, cg, range, red); break;
+        case 2: lin_mid_tile<K2, 2, SPLIT>(p, r0, rows, cg, range, red); break;
+        case 3: lin_mid_tile<K2, 3, SPLIT>(p, r0, rows, cg, range, red); break;
+        default: lin_mid_tile<K2, 4, SPLIT>(p, r0, rows, cg, range, red); break;
     }
+}
+
+// One wave per (row, 128 output columns): the ranges' accumulators added in range order, the codebook
+// map, C in fp16, Hadamard, fp16 svh product.
+__global__ __launch_bounds__(256) void lin_mid_epilogue_kernel(LinParams p)
+{
+    const int wid = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+    const int ncg = p.out / 128;
+    if (wid >= ncg * p.rows) return;
+    const int m = wid / ncg, cg = wid % ncg, lane = threadIdx.x & 63;
+    float sv[2];
+    lin_load_sv(p, cg, sv);
+    const float* src = p.part + (size_t)m * p.out + cg * 128 + lane_col(lane, 0);
+    const size_t stride = (size_t)p.rows * p.out;
+    float t[LIN_RANGES][2];
+#pragma unroll
+    for (int i = 0; i < LIN_RANGES; ++i) {
+        const float* q = src + (size_t)min(i, p.ks - 1) * stride;
+        t[i][0] = q[0];
+        t[i][1] = q[8];
+    }
+    const float xs = lin_row_total(p, m);
+    float v0 = t[0][0], v1 = t[0][1];
+#pragma unroll
+    for (int i = 1; i < LIN_RANGES; ++i)
+        if (i < p.ks) {
+            v0 += t[i][0];
+            v1 += t[i][1];
+        }
+    lin_store_row(p, m, cg, v0, v1, xs, sv);
+}
+
+// Calls of many rows: one workgroup per (256 rows, 128 output columns) over the whole k range, its
+// weights decoded once for the 256 rows (evamx_wide.hpp). Bound by the matrix cores and what feeds them:
+// the products alone take two thirds of its time at 8192 rows, without the decode it is 5% faster.
+// 2048 -> 7168 at 4 bpw, 8192 rows: 950 -> 356 us a call with its rotation (256 -> 676 TFLOP/s). The accumulators of the k-ranges that
+// lin_mid_kernel splits over workgroups are added in the same order, so the two give a row the same bits.
+// The epilogue runs on the accumulators where they are: a row's 128 columns lie on 16 lanes, whose
+// exchanges stay in a DPP row; the fp16 rows leave through LDS as whole 16-byte pieces.
+// Workgroup -> (row tile, column group). Workgroups are dispatched to the 8 XCDs round robin; each XCD
+// takes a contiguous share of the items, ordered by blocks of LW_GROUP row tiles with the tiles
+// fastest, so that the workgroups resident together on an XCD share LW_GROUP tiles' activations and a
+// few column groups' weights in its L2.
+constexpr int LW_GROUP = 4;
+__device__ __forceinline__ void lin_wide_item(int b, int nb, int tiles, int ncg, int& tile, int& cg)
+{
+    const int per = nb >> 3, rest = nb & 7, x = b & 7;
+    const int item = x * per + min(x, rest) + (b >> 3);
+    const int blk = item / (LW_GROUP * ncg), r = item - blk * LW_GROUP * ncg;
+    const int n = min(LW_GROUP, tiles - blk * LW_GROUP);
+    cg = r / n;
+    tile = blk * LW_GROUP + r % n;
+}
+
+constexpr int LW_MB = 2;
+constexpr int LW_WAVES = 8;
+constexpr int LW_ROWS = 16 * LW_MB * LW_WAVES;
+constexpr int LW_STRIDE = 136;                       // halves per staged output row (padded)
+
+template <int K2>
+__global__ __launch_bounds__(64 * LW_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void lin_wide_kernel(LinParams p)
+{
+    __shared__ union {
+        WideLds<LW_WAVES> w;
+        half_t y[LW_WAVES][16 * LW_MB][LW_STRIDE];
+    } lds;
+    __shared__ float xs[LW_WAVES][16 * LW_MB];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int g = lane >> 4;
+    const int ncg = p.out / 128, nch = p.in / 128;
+    int tile, cg;
+    lin_wide_item(blockIdx.x, gridDim.x, (p.rows + LW_ROWS - 1) / LW_ROWS, ncg, tile, cg);
+    const int r0 = tile * LW_ROWS + 16 * LW_MB * wave;
+    const __attribute__((address_space(1))) u32x4_t* arow[LW_MB];
+#pragma unroll
+    for (int mb = 0; mb < LW_MB; ++mb)                           // blocks past the call's: not stored
+        arow[mb] = (const __attribute__((address_space(1))) u32x4_t*)((const char*)p.xr + a_operand_offset(min(r0 / 16 + mb, (p.rows - 1) / 16), p.in)) + lane;
+    f32x4_t acc[LW_MB][8], tot[LW_MB][8];
+#pragma unroll
+    for (int mb = 0; mb < LW_MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb) acc[mb][nb] = tot[mb][nb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    int range = 0, stop = nch / p.ks;                            // the chunk after the range's last
+    wide_accumulate<K2, LW_MB, LW_WAVES>(p.trellis, p.out / 16, cg, 0, nch, arow, lds.w, acc, [&](int c) {
+        if (c + 1 != stop) return;
+#pragma unroll
+        for (int mb = 0; mb < LW_MB; ++mb)
+#pragma unroll
+            for (int nb = 0; nb < 8; ++nb) {
+                tot[mb][nb] += acc[mb][nb];
+                acc[mb][nb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        ++range;
+        stop = nch * (range + 1) / p.ks;
+    });
+    for (int i = 0; i < 16 * LW_MB; ++i) {
+        const float t = lin_row_total(p, min(r0 + i, p.rows - 1));
+        if (lane == 0) xs[wave][i] = t;
+    }
+    float sv[8];
+#pragma unroll
+    for (int nb = 0; nb < 8; ++nb) sv[nb] = h2f(p.svh[cg * 128 + mfma_col(lane, nb)]);
+    wave_lds_fence();
+#pragma unroll
+    for (int mb = 0; mb < LW_MB; ++mb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 16 * mb + 4 * g + r;
+            float v[8];
+#pragma unroll
+            for (int nb = 0; nb < 8; ++nb) v[nb] = h2f(f2h(mul1_affine(tot[mb][nb][r], xs[wave][row])));     // C in fp16
+            had128_acc(v, lane);
+#pragma unroll
+            for (int nb = 0; nb < 8; ++nb) lds.y[wave][row][mfma_col(lane, nb)] = f2h(h2f(f2h(v[nb])) * sv[nb]);
+        }
+    wave_lds_fence();
+    for (int i = lane; i < 16 * LW_MB * 16; i += 64) {
+        const int row = i >> 4, piece = i & 15;
+        if (r0 + row < p.rows)
+            *(u32x4_t*)(p.y + (size_t)(r0 + row) * p.out + cg * 128 + 8 * piece) = *(const u32x4_t*)&lds.y[wave][row][8 * piece];
+    }
+}
+
+// Kernel of a call of more than LIN_GEMV_ROWS rows. Wide tiles pay off once they fill the device, the
+// earlier the longer k is (a wide workgroup's fixed cost is its epilogue); below that the 64-row
+// workgroups over all ranges, and, when those are few, the ones of a range each (their partials cost
+// more the more tiles there are, the others' latency the longer k). us per call split / all ranges /
+// wide at 4 bpw, 2048 -> 7168: 64 rows 22 / 30 / 48, 256 rows 48 / 32 / 49, 512 rows 84 / 45 / 52, 1024
+// rows 161 / 79 / 58; 7168 -> 2048 (3.5 bpw): 256 rows 37 / 82 / 117, 512 rows 66 / 84 / 119, 1024 rows
+// 125 / 88 / 121, 2048 rows 241 / 141 / 128; 1024 -> 1024: 512 rows 20 / 24 / 38, 2048 rows 47 / 30 / 40,
+// 8192 rows 153 / 68 / 54.
+enum { LIN_SPLIT, LIN_FULL, LIN_WIDE };
+static int linear_kind(int rows, int in, int out)
+{
+    const long ncg = out / 128;
+    if ((rows + LW_ROWS - 1) / LW_ROWS * ncg >= 80 + 114688 / in) return LIN_WIDE;
+    // up to 32 rows and 1024 inputs the call is launches: one less (17.0 against 19.0 us)
+    if (rows <= 32 && in <= 1024) return LIN_FULL;
+    return (rows + LM_ROWS - 1) / LM_ROWS * ncg >= 80 + in / 76 ? LIN_FULL : LIN_SPLIT;
 }
 
 template <int K2>
-__device__ __forceinline__ void lin_mfma_rows(const LinParams& p, int r0, int rows, int cg, float (*red)[132])
+static void launch_rows_rate(const LinParams& p, int kind, hipStream_t stream)
 {
-    switch (__builtin_amdgcn_readfirstlane((rows + 15) >> 4)) {
-        case 1: lin_mfma_tile<K2, 1>(p, r0, rows, cg, red); break;
-        case 2: lin_mfma_tile<K2, 2>(p, r0, rows, cg, red); break;
-        case 3: lin_mfma_tile<K2, 3>(p, r0, rows, cg, red); break;
-        default: lin_mfma_tile<K2, 4>(p, r0, rows, cg, red); break;
+    const long ncg = p.out / 128;
+    const long tiles = (p.rows + LM_ROWS - 1) / LM_ROWS * ncg;
+    if (kind == LIN_WIDE) {
+        const dim3 grid((unsigned)((p.rows + LW_ROWS - 1) / LW_ROWS * ncg));
+        hipLaunchKernelGGL(lin_wide_kernel<K2>, grid, dim3(64 * LW_WAVES), 0, stream, p);
+    } else if (kind == LIN_FULL) {
+        hipLaunchKernelGGL((lin_mid_kernel<K2, false>), dim3((unsigned)tiles), dim3(64 * LM_WAVES), 0, stream, p);
+    } else {
+        hipLaunchKernelGGL((lin_mid_kernel<K2, true>), dim3((unsigned)(tiles * p.ks)), dim3(64 * LM_WAVES), 0, stream, p);
+        hipLaunchKernelGGL(lin_mid_epilogue_kernel, dim3((unsigned)((ncg * p.rows + 3) / 4)), dim3(256), 0, stream, p);
     }
 }
 
-__global__ __launch_bounds__(64 * LM_WAVES) void lin_mfma_kernel(LinParams p)
-{
-    __shared__ float red[64][132];      // padded rows: the partial stores hit 64 distinct banks
-    const int ncg = p.out / 128;
-    const int tile = blockIdx.x / ncg, cg = blockIdx.x % ncg;
-    const int r0 = 64 * tile, rows = p.rows - r0 < 64 ? p.rows - r0 : 64;
-    switch (p.k2) {
-        case 3: lin_mfma_rows<3>(p, r0, rows, cg, red); break;
-        case 4: lin_mfma_rows<4>(p, r0, rows, cg, red); break;
-        case 5: lin_mfma_rows<5>(p, r0, rows, cg, red); break;
-        case 6: lin_mfma_rows<6>(p, r0, rows, cg, red); break;
-        case 7: lin_mfma_rows<7>(p, r0, rows, cg, red); break;
-        case 8: lin_mfma_rows<8>(p, r0, rows, cg, red); break;
-        case 10: lin_mfma_rows<10>(p, r0, rows, cg, red); break;
-        default: break;                 // the rate is validated on the host
-    }
-}
-
-// k-split of a call: decode path, enough splits to fill the device once; MFMA path, one k-range
-// per wave of the workgroup. Both depend on in/out only.
+// k-split of a call: decode path, enough splits to fill the device once; beyond it the k-ranges. Both
+// depend on in/out only.
 int linear_ksplit(int rows, int in, int out)
 {
     const int ncg = out / 128, nch = in / 128;
-    if (rows > LIN_GEMV_ROWS) return nch < LM_WAVES ? nch : LM_WAVES;
+    if (rows > LIN_GEMV_ROWS) return nch < LIN_RANGES ? nch : LIN_RANGES;
     int ks = (4096 + ncg - 1) / ncg;
     if (ks > nch) ks = nch;
     if (ks < 1) ks = 1;
@@ -428,11 +633,11 @@ size_t linear_workspace(int rows, int in, int out, size_t* off_part, size_t* off
     if (off_sum) *off_sum = 0;
     if (off_part) *off_part = 0;
     if (rows > LIN_ROT_ROWS) {
-        o = al(o + (size_t)rows * in * 2);
+        o = al(o + (size_t)(rows > LIN_GEMV_ROWS ? (rows + 15) & ~15 : rows) * in * 2);
         if (off_sum) *off_sum = o;
         o = al(o + (size_t)rows * (in / 128) * 4);
     }
-    if (rows <= LIN_GEMV_ROWS) {
+    if (rows <= LIN_GEMV_ROWS || linear_kind(rows, in, out) == LIN_SPLIT) {
         if (off_part) *off_part = o;
         o = al(o + (size_t)linear_ksplit(rows, in, out) * rows * out * 4);
     }
@@ -456,26 +661,31 @@ int launch_linear(const void* x, int rows, int in, int out, const void* trellis,
     p.arrive = (unsigned long long*)ws;
     p.xr = rows > LIN_ROT_ROWS ? (half_t*)((char*)ws + off_xr) : nullptr;
     p.xsum = rows > LIN_ROT_ROWS ? (float*)((char*)ws + off_sum) : nullptr;
-    p.part = rows <= LIN_GEMV_ROWS ? (float*)((char*)ws + off_part) : nullptr;
-    if (rows > LIN_ROT_ROWS) {
+    p.part = rows <= LIN_GEMV_ROWS || linear_kind(rows, in, out) == LIN_SPLIT ? (float*)((char*)ws + off_part) : nullptr;
+    if (rows > LIN_GEMV_ROWS) {
+        hipLaunchKernelGGL(lin_rotate16_kernel, dim3((unsigned)((rows + 15) / 16 * (in / 128))), dim3(256), 0, stream, p);
+    } else if (rows > LIN_ROT_ROWS) {
         const long waves = (long)rows * (in / 128);
         hipLaunchKernelGGL(lin_rotate_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, p);
     }
-    if (rows > LIN_GEMV_ROWS) {
-        const long tiles = (rows + 63) / 64;
-        hipLaunchKernelGGL(lin_mfma_kernel, dim3((unsigned)(tiles * (out / 128))), dim3(64 * LM_WAVES), 0, stream, p);
-        return hipGetLastError() == hipSuccess ? 0 : -1;
-    }
+    int kind = rows > LIN_GEMV_ROWS ? linear_kind(rows, in, out) : -1;
+    if (kind == LIN_WIDE && ((uintptr_t)y & 15)) kind = LIN_FULL;      // its stores are 16 bytes wide
+#define EVAMX_LIN_RATE(K2)                                   \
+    case K2:                                                 \
+        if (kind >= 0) launch_rows_rate<K2>(p, kind, stream); \
+        else launch_gemv_rate<K2>(p, stream);                \
+        break
     switch (k2) {
-        case 3: launch_gemv_rate<3>(p, stream); break;
-        case 4: launch_gemv_rate<4>(p, stream); break;
-        case 5: launch_gemv_rate<5>(p, stream); break;
-        case 6: launch_gemv_rate<6>(p, stream); break;
-        case 7: launch_gemv_rate<7>(p, stream); break;
-        case 8: launch_gemv_rate<8>(p, stream); break;
-        case 10: launch_gemv_rate<10>(p, stream); break;
+        EVAMX_LIN_RATE(3);
+        EVAMX_LIN_RATE(4);
+        EVAMX_LIN_RATE(5);
+        EVAMX_LIN_RATE(6);
+        EVAMX_LIN_RATE(7);
+        EVAMX_LIN_RATE(8);
+        EVAMX_LIN_RATE(10);
         default: return -1;             // the rate is validated by the caller
     }
+#undef EVAMX_LIN_RATE
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

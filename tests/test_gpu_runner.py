@@ -114,3 +114,38 @@ def test_elinear_batch_invariant(dev):
     y17 = lin.forward(to_dev(x[84:], dev)).cpu().numpy()
     assert np.array_equal(y37.view(np.uint16), y101[20:57].view(np.uint16))
     assert np.array_equal(y17.view(np.uint16), y101[84:].view(np.uint16))
+
+
+@pytest.mark.parametrize("shape,K,counts", [
+    ((128, 128), 4, (17, 32, 33, 64, 65)),                     # one 128-chunk: one k-range
+    ((384, 256), 2.5, (17, 63, 129, 2048)),                    # fewer chunks than k-ranges
+    ((1152, 1024), 3, (33, 64, 192, 704, 1000, 6145)),         # uneven k-ranges; each kernel by size
+    ((1152, 1024), 5, (49, 6399)),
+    ((7168, 896), 1.5, (18, 300, 1920, 3600)),
+])
+def test_linear_row_kernels(dev, shape, K, counts):
+    """Above 16 rows a call takes one of three kernels by its size. Every row of every call has the bits
+    the row has in a 17-row call, at the edges of the 16-, 64- and 256-row tiles too; the 17-row calls are
+    held to the oracle."""
+    n_in, n_out = shape
+    rng = np.random.default_rng(n_in + n_out)
+    tr, suh, svh = synth.projection(rng, n_in, n_out, K, n_in ** -0.5)
+    from eva_amd import ops
+    from eva_amd.linear import build_linear
+    lin = build_linear(to_dev(suh, dev), to_dev(svh, dev), to_dev(tr, dev), device=dev, strict=False)
+    x = rng.standard_normal((max(counts), n_in)).astype(np.float16)
+    xd = to_dev(x, dev)
+    y17 = lin.forward(xd[:17].contiguous()).cpu().numpy()
+    ref = coop.exl3_linear(x[:17], tr, suh, svh, K)
+    assert rel_err_rows(y17.astype(np.float32), ref.astype(np.float32)) < TOL
+    for rows in counts:
+        y = lin.forward(xd[:rows].contiguous())
+        starts = sorted({0, max(0, rows - 17), max(0, rows // 2 - 8)} | {r for r in (56, 248) if r + 17 <= rows})
+        for r in starts:
+            want = lin.forward(xd[r:r + 17].contiguous())
+            assert torch.equal(y[r:r + 17][:rows - r].view(torch.int16), want[:min(17, rows - r)].view(torch.int16)), (rows, r)
+    # an output that starts off a 16-byte boundary
+    rows = max(counts)
+    buf = torch.zeros(rows * n_out + 1, dtype=torch.float16, device=dev)
+    ops.exl3_linear(xd, lin.trellis, lin.suh, lin.svh, K, out=buf[1:].view(rows, n_out))
+    assert torch.equal(buf[1:].view(rows, n_out).view(torch.int16), lin.forward(xd).view(torch.int16))
