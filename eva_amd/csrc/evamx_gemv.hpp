@@ -61,6 +61,90 @@ __device__ __forceinline__ void had128_pair(float& v0, float& v1, int lane)
     v1 *= R_SCALE;
 }
 
+// The same Hadamard with a chunk on 16 lanes, 8 consecutive elements a lane (a wave holds four chunks):
+// element bits 0-2 are in the lane; bits 3-6 pair lanes xor 1, 2, 7 and 8, each one DPP pattern of a
+// 16-lane row (xor 4 would take two and a select), so lane l holds the elements from 8 * oct_piece(l)
+// on. Same stages in the same order, so the results are bit-identical; 12 instructions an element
+// instead of 17, and a chunk's values move as 16-byte pieces.
+__device__ __forceinline__ int oct_piece(int lane)
+{
+    const int b2 = (lane >> 2) & 1;
+    return (((lane & 3) ^ (3 * b2)) | (lane & 12));
+}
+
+template <int CTRL>
+__device__ __forceinline__ void oct_stage(float (&v)[8], bool upper)
+{
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = dpp_f<CTRL>(v[i]) + (upper ? -v[i] : v[i]);
+}
+
+__device__ __forceinline__ void had128_oct(float (&v)[8], int lane)
+{
+    const int e = oct_piece(lane);
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+        const float a = v[i], c = v[i + 1];
+        v[i] = a + c;
+        v[i + 1] = a - c;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int i = (j & 1) + 4 * (j >> 1);
+        const float a = v[i], c = v[i + 2];
+        v[i] = a + c;
+        v[i + 2] = a - c;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = v[i], c = v[i + 4];
+        v[i] = a + c;
+        v[i + 4] = a - c;
+    }
+    oct_stage<0xB1>(v, e & 1);             // quad_perm [1,0,3,2]: lane xor 1
+    oct_stage<0x4E>(v, e & 2);             // quad_perm [2,3,0,1]: lane xor 2
+    oct_stage<0x141>(v, e & 4);            // row_half_mirror: lane xor 7
+    oct_stage<0x128>(v, e & 8);            // row_ror:8: lane xor 8
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] *= R_SCALE;
+}
+
+// Sum of a chunk's 8 values a lane after their rounding to fp16, in every lane of its 16.
+__device__ __forceinline__ float oct_sum(const half2_t (&r)[4])
+{
+    const half2_t one = {(half_t)1.0f, (half_t)1.0f};
+    float t = dot2(r[3], one, dot2(r[2], one, dot2(r[1], one, dot2(r[0], one, 0.0f))));
+    t += dpp_f<0xB1>(t);
+    t += dpp_f<0x4E>(t);
+    t += dpp_f<0x141>(t);
+    t += dpp_f<0x128>(t);
+    return t;
+}
+
+// 16-byte pieces of rows whose alignment is only that of their elements or of a dword (caller's
+// pointers); the compiler emits wide accesses where the hardware takes them.
+typedef uint32_t u32x4w __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4h __attribute__((ext_vector_type(4), aligned(2)));
+typedef float f32x4w __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ void oct_halves(const uint32_t (&w)[4], float (&v)[8])
+{
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const half2_t h = __builtin_bit_cast(half2_t, w[i]);
+        v[2 * i] = h2f(h.x);
+        v[2 * i + 1] = h2f(h.y);
+    }
+}
+
+// 8 fp16 values at p (2-byte aligned) as floats.
+__device__ __forceinline__ void oct_load_half(const half_t* p, float (&v)[8])
+{
+    const u32x4h w = *(const __attribute__((address_space(1))) u32x4h*)p;
+    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+    oct_halves(u, v);
+}
+
 // The codebook's affine map applied to a column's sums: sum_k x_k w_k = 0x1eee * sum_k x_k h_k +
 // 0xc931 * sum_k x_k, with one explicit fused multiply-add, so that no kernel's row count can change
 // how the compiler contracts it (a row's bits must not depend on its call's row count).

@@ -30,42 +30,66 @@ __device__ __forceinline__ void sum_splits(const float* const (&base)[N], size_t
     }
 }
 
+// One row's activation values (moe_act_kernel's operations) from its rotated gate and up values.
+__device__ __forceinline__ float act_value(bool shared, float L, float gg, float uu, float gs, float us, float ds)
+{
+    if (shared) {
+        // EXL3 linear outputs: fp16 after the rotation, fp16 product with svh; swiglu clamps the gate
+        // BEFORE SiLU; mid to fp16; fp16 product with the down suh
+        float gv = h2f(f2h(h2f(f2h(gg)) * gs));
+        float uv = h2f(f2h(h2f(f2h(uu)) * us));
+        if (L > 0.0f) {
+            // torch.clamp: a NaN stays NaN (fminf/fmaxf would return the limit)
+            uv = uv < -L ? -L : (uv > L ? L : uv);
+            gv = gv > L ? L : gv;
+        }
+        const float mid = h2f(f2h(silu_f(gv) * uv));
+        return h2f(f2h(mid * ds));
+    }
+    const float gv = gg * gs;
+    float uv = uu * us;
+    float x = silu_f(gv);
+    if (L != 0.0f) {
+        // fminf/fmaxf as the reference kernel: a NaN operand yields the limit
+        uv = fminf(fmaxf(uv, -L), L);
+        x = fminf(x, L);
+    }
+    return x * uv * ds;
+}
+
+// sigmoid(x_row . sh_gate_w) of a shared row (exl3_moe_coop_kernel.cuh:881-903), by one wave.
+__device__ __forceinline__ void shared_gate(const MoeParams& p, int row, int lane)
+{
+    const uint32_t* xw = (const uint32_t*)((const uint16_t*)p.x + (size_t)row * p.x_stride);
+    const uint32_t* ww = (const uint32_t*)p.sh_gate_w;
+    float d = 0.0f;
+    for (int i = lane; i < p.H / 2; i += 64) {
+        const uint32_t xv = xw[i];
+        const half2_t wv = __builtin_bit_cast(half2_t, ww[i]);
+        d = fmaf(x_elem(xv, 0, p.x_dtype), h2f(wv.x), d);
+        d = fmaf(x_elem(xv, 1, p.x_dtype), h2f(wv.y), d);
+    }
+    d = wave_sum(d);
+    if (lane == 0) p.gate_val[row] = 1.0f / (1.0f + __expf(-d));
+}
+
 // Activation epilogue: one wave per (grouped row o, 128-chunk a of I). Sums the gate/up
 // partials in fixed order, rounds to fp16 (gu_f32 = false), then exl3_moe_coop_kernel.cuh:
 // 784-805 for routed slots (act_gate with the clamp after SiLU) or the shared expert's EXL3
 // linear outputs + swiglu (model.py:450-452, kernels.py:213-217), and the down projection's
 // input rotation; writes act (fp16) and the chunk's sum.
-// REC (decode path): waves are (slot, chunk group), every slot's work resolved from its record
-// (inactive slots exit); otherwise (grouped row, chunk group) over the call's active rows.
-template <int CPW, bool REC>
+// REC (decode path): waves are (slot, chunk), every slot's work resolved from its record
+// (inactive slots exit); otherwise (grouped row, chunk) over the call's active rows (calls of up to
+// EVAMX_SMALL_ROWS rows; larger ones run moe_act_oct_kernel).
+template <bool REC>
 __global__ __launch_bounds__(256) void moe_act_kernel(MoeParams p)
 {
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     const int na = p.I / 128;
-    const int ng = na / CPW;                 // chunk groups per row (CPW divides na)
-    int o, a0;
-    if (!REC && p.act_class) {
-        // one size class of the MFMA tiles: wave -> (tile of the class, row of the tile up to the
-        // class's row bound, chunk group); rows past the tile's exit at once
-        const int cap = p.act_class == 1 ? EVAMX_SMALL_TILE_ROWS : EVAMX_TILE_ROWS;
-        const int n_small = __builtin_amdgcn_readfirstlane(p.meta[3]);
-        const int n_cls = p.act_class == 1 ? n_small : __builtin_amdgcn_readfirstlane(p.meta[0]) - n_small;
-        const int ti = wid / (cap * ng);
-        if (ti >= n_cls) return;
-        const int rem = wid - ti * cap * ng;
-        const int r = rem / ng;
-        a0 = (rem % ng) * CPW;
-        const int tile = __builtin_amdgcn_readfirstlane(p.act_class == 1 ? p.tiles[ti] : p.tiles[p.max_chunks - 1 - ti]);
-        const int* ch = p.chunks + 8 * tile;
-        if (r >= __builtin_amdgcn_readfirstlane(ch[2])) return;
-        o = __builtin_amdgcn_readfirstlane(ch[1]) + r;
-    } else {
-        const int n_rows = REC ? moe_nslot(p) : p.meta[1] + (p.has_shared ? p.T : 0);
-        if (wid >= n_rows * ng) return;
-        o = wid / ng;
-        a0 = (wid % ng) * CPW;
-    }
+    const int n_rows = REC ? moe_nslot(p) : p.meta[1] + (p.has_shared ? p.T : 0);
+    if (wid >= n_rows * na) return;
+    const int o = wid / na, a0 = wid % na;
     int s, Sg;
     bool shared;
     const half_t *g_svh, *u_svh, *d_suh;
@@ -89,126 +113,154 @@ __global__ __launch_bounds__(256) void moe_act_kernel(MoeParams p)
         Sg = ks_of_chunk(ks_gate_up(p, __builtin_amdgcn_readfirstlane(p.meta[2])),
                          __builtin_amdgcn_readfirstlane(p.slot_mult[s]));
     }
-    const float L = p.limit;
     const int nslot = moe_nslot(p);
-    if (shared && a0 == 0 && p.sh_gate_w) {
-        // gated shared expert: the row's scale sigmoid(x . w), fp32 dot of the fp16 row
-        // (exl3_moe_coop_kernel.cuh:881-903), for the combine stage
-        const int row = s - p.T * p.topk;
-        const uint32_t* xw = (const uint32_t*)((const uint16_t*)p.x + (size_t)row * p.x_stride);
-        const uint32_t* ww = (const uint32_t*)p.sh_gate_w;
-        float d = 0.0f;
-        for (int i = lane; i < p.H / 2; i += 64) {
-            const uint32_t xv = xw[i];
-            const half2_t wv = __builtin_bit_cast(half2_t, ww[i]);
-            d = fmaf(x_elem(xv, 0, p.x_dtype), h2f(wv.x), d);
-            d = fmaf(x_elem(xv, 1, p.x_dtype), h2f(wv.y), d);
-        }
-        d = wave_sum(d);
-        if (lane == 0) p.gate_val[row] = 1.0f / (1.0f + __expf(-d));
+    // gated shared expert: the row's scale, for the combine stage
+    if (shared && a0 == 0 && p.sh_gate_w) shared_gate(p, s - p.T * p.topk, lane);
+    // the scales and partial sums first, so their loads are in flight together
+    float gs[2], us[2], ds[2];
+    const float* base[4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int col = a0 * 128 + lane_col(lane, h);
+        gs[h] = h2f(g_svh[col]);
+        us[h] = h2f(u_svh[col]);
+        ds[h] = h2f(d_suh[col]);
+        base[h] = p.part_gu + (size_t)s * p.I + col;                          // gate
+        base[2 + h] = p.part_gu + (size_t)(nslot + s) * p.I + col;            // up
     }
-    // all chunks' scales and partial sums first, so their loads are in flight together
-    float g[CPW][2], u[CPW][2], gs[CPW][2], us[CPW][2], ds[CPW][2];
-    const float* base[4 * CPW];
+    float sums[4];
+    sum_splits<4, 8>(base, (size_t)2 * nslot * p.I, Sg, sums);
+    float gg[2], uu[2];
 #pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int col = (a0 + c) * 128 + lane_col(lane, h);
-            gs[c][h] = h2f(g_svh[col]);
-            us[c][h] = h2f(u_svh[col]);
-            ds[c][h] = h2f(d_suh[col]);
-            base[4 * c + h] = p.part_gu + (size_t)s * p.I + col;                          // gate
-            base[4 * c + 2 + h] = p.part_gu + (size_t)(nslot + s) * p.I + col;            // up
-        }
+    for (int h = 0; h < 2; ++h) {
+        gg[h] = h2f(f2h(sums[h]));         // GEMV output stored as fp16 (gu_f32 = false)
+        uu[h] = h2f(f2h(sums[2 + h]));
     }
-    float sums[4 * CPW];
-    sum_splits<4 * CPW, CPW == 1 ? 8 : 2>(base, (size_t)2 * nslot * p.I, Sg, sums);
+    had128_lane(gg[0], gg[1], lane);
+    had128_lane(uu[0], uu[1], lane);
+    float av[2];
 #pragma unroll
-    for (int c = 0; c < CPW; ++c)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            g[c][h] = sums[4 * c + h];
-            u[c][h] = sums[4 * c + 2 + h];
-        }
-#pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-        float gg[2], uu[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            gg[h] = h2f(f2h(g[c][h]));     // GEMV output stored as fp16 (gu_f32 = false)
-            uu[h] = h2f(f2h(u[c][h]));
-        }
-        had128_lane(gg[0], gg[1], lane);
-        had128_lane(uu[0], uu[1], lane);
-        float av[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            if (shared) {
-                // EXL3 linear outputs: fp16 after the rotation, fp16 product with svh; swiglu
-                // clamps the gate BEFORE SiLU; mid to fp16; fp16 product with the down suh
-                float gv = h2f(f2h(h2f(f2h(gg[h])) * gs[c][h]));
-                float uv = h2f(f2h(h2f(f2h(uu[h])) * us[c][h]));
-                if (L > 0.0f) {
-                    // torch.clamp: a NaN stays NaN (fminf/fmaxf would return the limit)
-                    uv = uv < -L ? -L : (uv > L ? L : uv);
-                    gv = gv > L ? L : gv;
-                }
-                const float mid = h2f(f2h(silu_f(gv) * uv));
-                av[h] = h2f(f2h(mid * ds[c][h]));
-            } else {
-                const float gv = gg[h] * gs[c][h];
-                float uv = uu[h] * us[c][h];
-                float x = silu_f(gv);
-                if (L != 0.0f) {
-                    // fminf/fmaxf as the reference kernel: a NaN operand yields the limit
-                    uv = fminf(fmaxf(uv, -L), L);
-                    x = fminf(x, L);
-                }
-                av[h] = x * uv * ds[c][h];
-            }
-        }
-        had128_lane(av[0], av[1], lane);
-        half_t* dst = p.act + (size_t)s * p.I + (a0 + c) * 128;
-        const half_t r0 = f2h(av[0]), r1 = f2h(av[1]);
-        dst[lane_col(lane, 0)] = r0;
-        dst[lane_col(lane, 1)] = r1;
-        const float sum = wave_sum(h2f(r0) + h2f(r1));
-        if (lane == 0) p.actsum[(size_t)s * na + a0 + c] = sum;
+    for (int h = 0; h < 2; ++h) av[h] = act_value(shared, p.limit, gg[h], uu[h], gs[h], us[h], ds[h]);
+    had128_lane(av[0], av[1], lane);
+    half_t* dst = p.act + (size_t)s * p.I + a0 * 128;
+    const half_t r0 = f2h(av[0]), r1 = f2h(av[1]);
+    dst[lane_col(lane, 0)] = r0;
+    dst[lane_col(lane, 1)] = r1;
+    const float sum = wave_sum(h2f(r0) + h2f(r1));
+    if (lane == 0) p.actsum[(size_t)s * na + a0] = sum;
+}
+
+// 8 consecutive fp32 partials at b (16-byte aligned), splits q < S `stride` apart added in order.
+__device__ __forceinline__ void oct_partials(const float* b, size_t stride, int S, float (&v)[8])
+{
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    const __attribute__((address_space(1))) f32x4* q = (const __attribute__((address_space(1))) f32x4*)b;
+    f32x4 lo = q[0], hi = q[1];
+    for (int i = 1; i < S; ++i) {
+        q = (const __attribute__((address_space(1))) f32x4*)(b + (size_t)i * stride);
+        lo += q[0];
+        hi += q[1];
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        v[i] = lo[i];
+        v[4 + i] = hi[i];
+    }
+}
+
+// The activation stage of a large call, 16 lanes a chunk: a wave takes four 128-chunks of a grouped row.
+// Same operations as moe_act_kernel on the MFMA path. Bound by the partials it reads (3001 tokens, both size
+// classes beside the other class's GEMMs: 646 -> 252 us; one wave with 4-byte loads before).
+__global__ __launch_bounds__(256) void moe_act_oct_kernel(MoeParams p)
+{
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+    const int na = p.I / 128, ng = (na + 3) / 4, slots = p.T * p.topk;
+    int o, q;
+    if (p.act_class) {
+        // one size class of the MFMA tiles: wave -> (tile of the class, row of the tile up to the
+        // class's row bound, chunk group); rows past the tile's exit at once
+        const int cap = p.act_class == 1 ? EVAMX_SMALL_TILE_ROWS : EVAMX_TILE_ROWS;
+        const int n_small = __builtin_amdgcn_readfirstlane(p.meta[3]);
+        const int n_cls = p.act_class == 1 ? n_small : __builtin_amdgcn_readfirstlane(p.meta[0]) - n_small;
+        const int ti = wid / (cap * ng);
+        if (ti >= n_cls) return;
+        const int rem = wid - ti * cap * ng, r = rem / ng;
+        q = rem % ng;
+        const int tile = __builtin_amdgcn_readfirstlane(p.act_class == 1 ? p.tiles[ti] : p.tiles[p.max_chunks - 1 - ti]);
+        const int* ch = p.chunks + 8 * tile;
+        if (r >= __builtin_amdgcn_readfirstlane(ch[2])) return;
+        o = __builtin_amdgcn_readfirstlane(ch[1]) + r;
+    } else {
+        if (wid >= (p.meta[1] + (p.has_shared ? p.T : 0)) * ng) return;
+        o = wid / ng;
+        q = wid % ng;
+    }
+    const int s = __builtin_amdgcn_readfirstlane(p.order[o]);
+    const int e = s < slots ? __builtin_amdgcn_readfirstlane(p.local[s]) : -1;
+    const bool shared = e < 0;
+    const half_t* g_svh = (const half_t*)expert_ptr(p, e, EVAMX_TBL_G_SVH);
+    const half_t* u_svh = (const half_t*)expert_ptr(p, e, EVAMX_TBL_U_SVH);
+    const half_t* d_suh = (const half_t*)expert_ptr(p, e, EVAMX_TBL_D_SUH);
+    const int S = ks_of_chunk(ks_gate_up(p, __builtin_amdgcn_readfirstlane(p.meta[2])),
+                              __builtin_amdgcn_readfirstlane(p.slot_mult[s]));
+    if (shared && q == 0 && p.sh_gate_w) shared_gate(p, s - slots, lane);
+    const int c = 4 * q + (lane >> 4);
+    if (c >= na) return;                                  // whole 16-lane rows: the exchanges stay inside one
+    const int nslot = moe_nslot(p), col = 128 * c + 8 * oct_piece(lane);
+    const size_t stride = (size_t)2 * nslot * p.I;
+    float g[8], u[8], gs[8], us[8], ds[8];
+    oct_load_half(g_svh + col, gs);
+    oct_load_half(u_svh + col, us);
+    oct_load_half(d_suh + col, ds);
+    oct_partials(p.part_gu + (size_t)s * p.I + col, stride, S, g);
+    oct_partials(p.part_gu + (size_t)(nslot + s) * p.I + col, stride, S, u);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        g[i] = h2f(f2h(g[i]));                            // GEMV output stored as fp16 (gu_f32 = false)
+        u[i] = h2f(f2h(u[i]));
+    }
+    had128_oct(g, lane);
+    had128_oct(u, lane);
+    float av[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) av[i] = act_value(shared, p.limit, g[i], u[i], gs[i], us[i], ds[i]);
+    had128_oct(av, lane);
+    half2_t r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = half2_t{f2h(av[2 * i]), f2h(av[2 * i + 1])};
+    *(u32x4*)(p.act + (size_t)s * p.I + col) = u32x4{__builtin_bit_cast(uint32_t, r[0]), __builtin_bit_cast(uint32_t, r[1]),
+                                                     __builtin_bit_cast(uint32_t, r[2]), __builtin_bit_cast(uint32_t, r[3])};
+    const float sum = oct_sum(r);
+    if ((lane & 15) == 0) p.actsum[(size_t)s * na + c] = sum;
 }
 
 // The activation stage for the rows of one size class of MFMA tiles (cls 1: tiles of at most 16
 // rows, cls 2: larger), calls of more than 16 tokens.
 void launch_act_class(const MoeParams& p, int cls, hipStream_t stream)
 {
-    const int na = p.I / 128;
+    const int ng = (p.I / 128 + 3) / 4;
     MoeParams q = p;
     q.act_class = cls;
     const long cap = cls == 1 ? EVAMX_SMALL_TILE_ROWS : EVAMX_TILE_ROWS;
-    if (p.T > EVAMX_SMALL_ROWS && na % 4 == 0) {
-        const long waves = (long)p.max_chunks * cap * (na / 4);
-        launch_timed(moe_act_kernel<4, false>, dim3((unsigned)((waves + 3) / 4)), dim3(256), stream, nullptr, nullptr, q);
-    } else {
-        const long waves = (long)p.max_chunks * cap * na;
-        launch_timed(moe_act_kernel<1, false>, dim3((unsigned)((waves + 3) / 4)), dim3(256), stream, nullptr, nullptr, q);
-    }
+    const long waves = (long)p.max_chunks * cap * ng;
+    launch_timed(moe_act_oct_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), stream, nullptr, nullptr, q);
 }
 
-// Activation launch: one wave per (row, chunk) for small batches (latency), per (row, 4 chunks)
-// for large ones (the row's slot, expert and pointers resolved once).
+// Activation launch: one wave per (row, chunk) for small batches (latency), per (row, 4 chunks) for
+// large ones.
 void launch_act(const MoeParams& p, int nslot, hipStream_t stream, hipEvent_t start, hipEvent_t stop)
 {
     const int na = p.I / 128;
     if (!p.mfma) {
         const int waves = nslot * na;
-        launch_timed(moe_act_kernel<1, true>, dim3((waves + 3) / 4), dim3(256), stream, start, stop, p);
-    } else if (p.T > EVAMX_SMALL_ROWS && na % 4 == 0) {
-        const int waves = nslot * (na / 4);
-        launch_timed(moe_act_kernel<4, false>, dim3((waves + 3) / 4), dim3(256), stream, start, stop, p);
+        launch_timed(moe_act_kernel<true>, dim3((waves + 3) / 4), dim3(256), stream, start, stop, p);
+    } else if (p.T > EVAMX_SMALL_ROWS) {
+        const int waves = nslot * ((na + 3) / 4);
+        launch_timed(moe_act_oct_kernel, dim3((waves + 3) / 4), dim3(256), stream, start, stop, p);
     } else {
         const int waves = nslot * na;
-        launch_timed(moe_act_kernel<1, false>, dim3((waves + 3) / 4), dim3(256), stream, start, stop, p);
+        launch_timed(moe_act_kernel<false>, dim3((waves + 3) / 4), dim3(256), stream, start, stop, p);
     }
 }
 
@@ -350,79 +402,89 @@ __global__ __launch_bounds__(64 * EVAMX_COMBINE_WAVES) void moe_combine_kernel(M
 }
 
 // The same reduction for large batches, where throughput matters more than the latency of one
-// token: one wave per (token, CGW groups of 128 columns) walks the token's items in slot order
-// (shared expert last), COMBINE_BATCH items at a time: it reads their metadata (local expert,
-// split count, weight, svh pointer) once for its CGW column groups, then for each column group
-// issues the items' loads together and adds them in slot order. Same operations in the same order
-// per column as moe_combine_kernel, so the two give identical results.
-constexpr int COMBINE_BATCH = 4;      // 9 (all of DSv3's items at once) was slower: 512 tokens 88.3-88.8 -> 90.9-91.5 us
+// token: one wave per (token, four 128-column groups, 16 lanes each) walks the token's items in slot
+// order (shared expert last), COMBINE_BATCH items at a time: it reads their metadata (local expert,
+// split count, weight, svh pointer), issues the items' loads together and adds them in slot order. Same
+// operations in the same order per column as moe_combine_kernel, so the two give identical results.
+// Bound by the partials it reads (512 tokens mixed: 82 -> 38 us, 3001 tokens: 496 -> 187; one
+// wave per two column groups with 4-byte loads before).
+constexpr int COMBINE_BATCH = 3;
 
-template <int CGW>
 __global__ __launch_bounds__(256) void moe_combine_rows_kernel(MoeParams p)
 {
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
-    const int ngw = p.H / 128 / CGW;                 // column-group blocks per token (CGW divides H/128)
-    if (wid >= p.T * ngw) return;
-    const int row = wid / ngw, cg0 = (wid - row * ngw) * CGW;
-    const int slots = p.T * p.topk;
+    const int ncg = p.H / 128, nq = (ncg + 3) / 4;
+    if (wid >= p.T * nq) return;
+    const int row = wid / nq, cg = 4 * (wid - row * nq) + (lane >> 4);
+    const int slots = p.T * p.topk, nslot = moe_nslot(p);
     const KSplit kd = ks_down(p, __builtin_amdgcn_readfirstlane(p.meta[2]));
     const int nitems = p.topk + (p.has_shared ? 1 : 0);
-    float o[CGW][2];
+    if (cg >= ncg) return;                                // whole 16-lane rows: the exchanges stay inside one
+    const int col = 128 * cg + 8 * oct_piece(lane);
+    float o[8];
 #pragma unroll
-    for (int c = 0; c < CGW; ++c) o[c][0] = o[c][1] = 0.0f;
+    for (int i = 0; i < 8; ++i) o[i] = 0.0f;
     for (int b = 0; b < nitems; b += COMBINE_BATCH) {
-        int sk[COMBINE_BATCH], le[COMBINE_BATCH], S[COMBINE_BATCH];
-        float w[COMBINE_BATCH];
         const half_t* svh[COMBINE_BATCH];
+        float w[COMBINE_BATCH], v[COMBINE_BATCH][8], sv[COMBINE_BATCH][8];
 #pragma unroll
         for (int j = 0; j < COMBINE_BATCH; ++j) {
             const int k = b + j;
             const bool shared = k == p.topk;
-            sk[j] = shared ? slots + row : row * p.topk + k;
-            le[j] = -2;                                   // -2: past the items
-            svh[j] = nullptr;
-            if (k < nitems) {
-                le[j] = shared ? -1 : __builtin_amdgcn_readfirstlane(p.local[sk[j]]);
-                S[j] = ks_of_chunk(kd, __builtin_amdgcn_readfirstlane(p.slot_mult[sk[j]]));
-                w[j] = shared ? 1.0f : h2f(p.rw16[sk[j]]);
-                if (le[j] >= 0 || (shared && le[j] == -1))
-                    svh[j] = shared ? (const half_t*)p.sh_ptr[EVAMX_TBL_D_SVH]
-                                    : (const half_t*)p.tables[(size_t)EVAMX_TBL_D_SVH * p.tbl_stride + le[j]];
-            }
+            svh[j] = nullptr;                                  // past the items, or an inactive slot
+            if (k >= nitems) continue;
+            const int sk = shared ? slots + row : row * p.topk + k;
+            const int le = shared ? -1 : __builtin_amdgcn_readfirstlane(p.local[sk]);
+            if (!shared && le < 0) continue;
+            svh[j] = (const half_t*)uniform_u64(shared ? (uint64_t)p.sh_ptr[EVAMX_TBL_D_SVH]
+                                                       : (uint64_t)p.tables[(size_t)EVAMX_TBL_D_SVH * p.tbl_stride + le]);
+            w[j] = shared ? 1.0f : h2f(p.rw16[sk]);
+            const int S = ks_of_chunk(kd, __builtin_amdgcn_readfirstlane(p.slot_mult[sk]));
+            oct_load_half(svh[j] + col, sv[j]);
+            oct_partials(p.part_d + (size_t)sk * p.H + col, (size_t)nslot * p.H, S, v[j]);
         }
 #pragma unroll
-        for (int c = 0; c < CGW; ++c) {
-            const int cg = cg0 + c;
-            const int col0 = cg * 128 + lane_col(lane, 0), col1 = cg * 128 + lane_col(lane, 1);
-            float v[COMBINE_BATCH][2], sv[COMBINE_BATCH][2];
+        for (int j = 0; j < COMBINE_BATCH; ++j) {
+            if (!svh[j]) continue;
+            const bool shared = b + j == p.topk;
+            if (shared) {
 #pragma unroll
-            for (int j = 0; j < COMBINE_BATCH; ++j) {
-                if (svh[j]) {
-                    sum_partials(p, sk[j], cg, lane, S[j], v[j]);
-                    sv[j][0] = h2f(svh[j][col0]);
-                    sv[j][1] = h2f(svh[j][col1]);
-                }
+                for (int i = 0; i < 8; ++i) v[j][i] = h2f(f2h(v[j][i]));
             }
+            had128_oct(v[j], lane);
+            const float gv = shared && p.sh_gate_w ? p.gate_val[row] : 1.0f;
 #pragma unroll
-            for (int j = 0; j < COMBINE_BATCH; ++j) {
-                if (svh[j]) {
-                    const bool shared = b + j == p.topk;
-                    combine_item(shared, w[j], sv[j][0], sv[j][1], v[j], lane);
-                    if (shared && p.sh_gate_w) {
-                        const float gv = p.gate_val[row];
-                        v[j][0] = gv * v[j][0];
-                        v[j][1] = gv * v[j][1];
-                    }
-                    o[c][0] = o[c][0] + v[j][0];
-                    o[c][1] = o[c][1] + v[j][1];
+            for (int i = 0; i < 8; ++i) {
+                float t;
+                if (shared) {
+                    t = h2f(f2h(h2f(f2h(v[j][i])) * sv[j][i]));
+                    if (p.sh_gate_w) t = gv * t;
+                } else {
+                    t = w[j] * (v[j][i] * sv[j][i]);
                 }
+                o[i] = o[i] + t;
             }
         }
     }
+    if (p.out) {
+        float* dst = p.out + (size_t)row * p.out_stride + col;
+        *(f32x4w*)dst = f32x4w{o[0], o[1], o[2], o[3]};
+        *(f32x4w*)(dst + 4) = f32x4w{o[4], o[5], o[6], o[7]};
+    }
+    if (p.residual) {
+        // h = bf16(h + bf16(y)), as combine_store
+        u32x4h* h = (u32x4h*)(p.residual + (size_t)row * p.residual_stride + col);
+        const u32x4h hv = *h;
+        u32x4h r;
 #pragma unroll
-    for (int c = 0; c < CGW; ++c)
-        combine_store(p, row, (cg0 + c) * 128 + lane_col(lane, 0), (cg0 + c) * 128 + lane_col(lane, 1), o[c][0], o[c][1]);
+        for (int i = 0; i < 4; ++i) {
+            const uint16_t lo = bf16_bits(bf16_value((uint16_t)hv[i]) + bf16_value(bf16_bits(o[2 * i])));
+            const uint16_t hi = bf16_bits(bf16_value((uint16_t)(hv[i] >> 16)) + bf16_value(bf16_bits(o[2 * i + 1])));
+            r[i] = (uint32_t)lo | (uint32_t)hi << 16;
+        }
+        *h = r;
+    }
 }
 
 void launch_combine(const MoeParams& p, hipStream_t stream, hipEvent_t start, hipEvent_t stop)
@@ -435,11 +497,7 @@ void launch_combine(const MoeParams& p, hipStream_t stream, hipEvent_t start, hi
         else
             launch_timed(moe_combine_kernel<false>, dim3(p.T * (p.H / 128)), dim3(64 * nw), stream, start, stop, p);
     } else {
-        // two column groups per wave: 512 tokens 90.6 -> 88.1 us (four: 100 us, too few waves)
-        if ((p.H / 128) % 2 == 0)
-            launch_timed(moe_combine_rows_kernel<2>, dim3((p.T * (p.H / 256) + 3) / 4), dim3(256), stream, start, stop, p);
-        else
-            launch_timed(moe_combine_rows_kernel<1>, dim3((p.T * (p.H / 128) + 3) / 4), dim3(256), stream, start, stop, p);
+        launch_timed(moe_combine_rows_kernel, dim3((p.T * ((p.H / 128 + 3) / 4) + 3) / 4), dim3(256), stream, start, stop, p);
     }
 }
 

@@ -560,13 +560,57 @@ __global__ __launch_bounds__(64 * GROUP_WAVES) void moe_group_kernel(MoeParams p
     }
 }
 
+// Input rotations of a large call (rotate_chunks' operations, 16 lanes a chunk): a wave takes four
+// 128-chunks of a grouped row and rotates them for gate and up, so x is read and converted once.
+// Bound by the butterflies' vector instructions, then by the rows it writes (512 tokens mixed: 89 ->
+// 58 us, 3001 tokens: 499 -> 319).
 constexpr int EVAMX_ROTATE_BLOCKS = 2048;
 
 __global__ __launch_bounds__(256) void moe_rotate_kernel(MoeParams p)
 {
     const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
-    rotate_rows(p, p.order, p.local, p.meta[1] + (p.has_shared ? p.T : 0), w, gridDim.x * 4, lane);
+    const int w0 = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+    const int n_rows = p.meta[1] + (p.has_shared ? p.T : 0);
+    const int nch = p.H / 128, nq = (nch + 3) / 4, slots = p.T * p.topk;
+    const int piece = oct_piece(lane);
+    for (int it = w0; it < n_rows * nq; it += gridDim.x * 4) {
+        const int o = it / nq, c = 4 * (it - o * nq) + (lane >> 4);
+        const int s = __builtin_amdgcn_readfirstlane(p.order[o]);
+        const bool shared = s >= slots;
+        const int e = shared ? -1 : __builtin_amdgcn_readfirstlane(p.local[s]);
+        const int row = shared ? s - slots : s / p.topk;
+        if (c >= nch) continue;                           // whole 16-lane rows: the exchanges stay inside one
+        const int k = 128 * c + 8 * piece;
+        const uint64_t pg = uniform_u64(shared ? (uint64_t)p.sh_ptr[EVAMX_TBL_G_SUH] : (uint64_t)p.tables[(size_t)EVAMX_TBL_G_SUH * p.tbl_stride + e]);
+        const uint64_t pu = uniform_u64(shared ? (uint64_t)p.sh_ptr[EVAMX_TBL_U_SUH] : (uint64_t)p.tables[(size_t)EVAMX_TBL_U_SUH * p.tbl_stride + e]);
+        const u32x4w xw = *(const __attribute__((address_space(1))) u32x4w*)((const uint16_t*)p.x + (size_t)row * p.x_stride + k);
+        float sg[8], su[8], x[8];
+        oct_load_half((const half_t*)pg + k, sg);
+        oct_load_half((const half_t*)pu + k, su);
+        const uint32_t xu[4] = {xw.x, xw.y, xw.z, xw.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = x_elem(xu[i >> 1], i & 1, p.x_dtype);
+#pragma unroll
+        for (int proj = 0; proj < 2; ++proj) {
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                // shared expert: fp16 product (hadamard_inner.cuh:109-115); routed: fp32 product
+                v[i] = x[i] * (proj == 0 ? sg[i] : su[i]);
+                if (shared) v[i] = h2f(f2h(v[i]));
+            }
+            had128_oct(v, lane);
+            half2_t r[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r[i] = half2_t{f2h(v[2 * i]), f2h(v[2 * i + 1])};
+            const size_t at = (size_t)proj * p.nslot_max + s;
+            const u32x4 out = {__builtin_bit_cast(uint32_t, r[0]), __builtin_bit_cast(uint32_t, r[1]),
+                               __builtin_bit_cast(uint32_t, r[2]), __builtin_bit_cast(uint32_t, r[3])};
+            *(u32x4*)(p.xr + at * p.H + k) = out;
+            const float sum = oct_sum(r);
+            if ((lane & 15) == 0) p.xsum[at * nch + c] = sum;
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
