@@ -239,6 +239,18 @@ __host__ __device__ __forceinline__ KSplit ks_down(const MoeParams& p, int units
 
 __host__ __device__ __forceinline__ int chunk_rows_of(const MoeParams& p) { return p.chunk_rows > 0 ? p.chunk_rows : EVAMX_CHUNK; }
 
+// The most MFMA tiles of a size class (1: at most 16 rows, 2: more) that a call of more than
+// EVAMX_SMALL_TILE_ROWS tokens can have: an expert has one tile of at most 16 rows at most, its last, and a
+// larger one holds 17 rows or more. Launches are sized by it; the workspace's tile bound is ten times as
+// large at 3000 tokens, and a workgroup without work still takes its turn behind the other class's.
+inline long moe_class_tiles(const MoeParams& p, int cls)
+{
+    const long slots = (long)p.T * p.topk;
+    const long n = cls == 1 ? (slots < p.n_local ? slots : p.n_local) + (p.has_shared ? 1 : 0)
+                            : slots / (EVAMX_SMALL_TILE_ROWS + 1) + (p.has_shared ? (p.T + EVAMX_TILE_ROWS - 1) / EVAMX_TILE_ROWS : 0);
+    return n < p.max_chunks ? n : p.max_chunks;
+}
+
 int moe_launch(MoeParams& p, hipStream_t stream, void* const* events = nullptr);
 // Stage launches of moe_launch, one translation unit each (moe_prepare.hip, moe_gate_up*.hip,
 // moe_down.hip, moe_epilogue.hip). start/stop: events that take the first kernel's start and the

@@ -243,7 +243,8 @@ void launch_act_class(const MoeParams& p, int cls, hipStream_t stream)
     MoeParams q = p;
     q.act_class = cls;
     const long cap = cls == 1 ? EVAMX_SMALL_TILE_ROWS : EVAMX_TILE_ROWS;
-    const long waves = (long)p.max_chunks * cap * ng;
+    const long waves = moe_class_tiles(p, cls) * cap * ng;
+    if (waves == 0) return;
     launch_timed(moe_act_oct_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), stream, nullptr, nullptr, q);
 }
 

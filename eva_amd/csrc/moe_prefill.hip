@@ -223,23 +223,22 @@ const SideStream* side_stream(hipStream_t stream)
     return &ss;
 }
 
-// The largest possible item count of one projection stage: the workspace's tile bound times the
-// largest split (an automatic split fills one resident round; gate/up: up to two, see ks_gate_up).
-static long mfma_items(const MoeParams& p, int which)
+// The largest possible item count of one projection stage for at most `tiles` tiles: times the largest
+// split (an automatic split fills one resident round; gate/up: up to two, see ks_gate_up).
+static long mfma_items(const MoeParams& p, int which, long tiles)
 {
     const int ncg = which == 0 ? p.I / 128 : p.H / 128;
     const int kreq = which == 0 ? p.ks_gu : p.ks_d;
     const long per_tile = (long)(which == 0 ? 2 * ncg : ncg);
     const long auto_items = (long)(which == 0 ? 2 : 1) * p.gemv_waves + per_tile;
-    return kreq > 0 ? (long)p.max_chunks * per_tile * kreq
-                    : (p.max_chunks * per_tile > auto_items ? (long)p.max_chunks * per_tile : auto_items);
+    return kreq > 0 ? tiles * per_tile * kreq : (tiles * per_tile > auto_items ? tiles * per_tile : auto_items);
 }
 
 // Grid of one projection stage in the single-wave form: enough workgroups for mfma_items (a
 // multiple of 8); workgroups past the call's items exit at once.
-static dim3 mfma_grid(const MoeParams& p, int which)
+static dim3 mfma_grid(const MoeParams& p, int which, long tiles)
 {
-    const long blocks = (mfma_items(p, which) + MF_WAVES - 1) / MF_WAVES;
+    const long blocks = (mfma_items(p, which, tiles) + MF_WAVES - 1) / MF_WAVES;
     return dim3((unsigned)((blocks + 7) & ~7L));
 }
 
@@ -247,7 +246,9 @@ int launch_mfma_class(const MoeParams& p, int which, int cls, hipStream_t stream
 {
     MoeParams q = p;
     q.force_split = 1;
-    const dim3 grid = mfma_grid(p, which), block(64 * MF_WAVES);
+    const long tiles = moe_class_tiles(p, cls);
+    if (tiles == 0) return 0;
+    const dim3 grid = mfma_grid(p, which, tiles), block(64 * MF_WAVES);
     if (cls == 1)
         launch_timed(which == 0 ? moe_gate_up_mfma_kernel<1> : moe_down_mfma_kernel<1>, grid, block, stream, nullptr, nullptr, q);
     else
@@ -263,7 +264,6 @@ int launch_mfma(const MoeParams& p, int which, hipStream_t stream, hipEvent_t st
     const int kreq = which == 0 ? p.ks_gu : p.ks_d;
     const int kmax = which == 0 ? p.ks_gu_max : p.ks_d_max;
     const long per_tile = (long)(which == 0 ? 2 * ncg : ncg);
-    const long items = mfma_items(p, which);
     // tiles of at most 16 rows run in the 16-row kernel (4 waves per SIMD, progress priorities),
     // larger ones in the 64-row kernel; up to 16 tokens every tile is a small one
     // The small-tile launch is skipped when the split can never happen: at most one tile per
@@ -275,7 +275,7 @@ int launch_mfma(const MoeParams& p, int which, hipStream_t stream, hipEvent_t st
     const bool may_split = max_small * per_tile * s_max >= 3L * (p.gemv_waves * 3 / 4);
     auto k16 = which == 0 ? moe_gate_up_mfma_kernel<1> : moe_down_mfma_kernel<1>;
     auto k64 = which == 0 ? moe_gate_up_mfma_kernel<4> : moe_down_mfma_kernel<4>;
-    const dim3 grid = mfma_grid(p, which), block(64 * MF_WAVES);
+    const dim3 grid = mfma_grid(p, which, p.max_chunks), block(64 * MF_WAVES);
     if (const SideStream* side = p.T > EVAMX_SMALL_TILE_ROWS && p.side_ok ? side_stream(stream) : nullptr) {
         // the tiles of at most 16 rows in the 16-row kernel on the side stream, concurrently with
         // the larger ones in the 64-row kernel on the caller's stream: each fills the other's
