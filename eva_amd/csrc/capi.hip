@@ -214,7 +214,7 @@ extern "C" int evamx_exl3_dequant(const void* trellis, int in_features, int out_
     EVAMX_REQUIRE(k2 > 0, "evamx_exl3_dequant: unsupported bit rate %g", (double)bits);
     EVAMX_REQUIRE(in_features >= 16 && out_features >= 16 && in_features % 16 == 0 && out_features % 16 == 0,
                   "evamx_exl3_dequant: in/out (%d, %d) must be positive multiples of 16", in_features, out_features);
-    launch_dequant(trellis, in_features, out_features, k2, w_fp16, false, (hipStream_t)stream);
+    launch_dequant(trellis, in_features, out_features, k2, w_fp16, (hipStream_t)stream);
     return launched("dequant");
 }
 

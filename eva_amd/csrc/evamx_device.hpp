@@ -47,19 +47,8 @@ __device__ __forceinline__ uint32_t mul1_hash(uint32_t r)
     return p;
 }
 
-// Two decoded weights (fp16, bit-exact MUL1 decode) from two hashes:
-// h = fp16_bits(0x6400 + bytesum) = 1024 + bytesum, w = fma_fp16(h, 0x1eee, 0xc931).
-__device__ __forceinline__ half2_t mul1_pair(uint32_t p0, uint32_t p1)
-{
-    uint32_t s = __builtin_amdgcn_sad_u8(p0, 0u, 0x64006400u);
-    s = __builtin_amdgcn_sad_hi_u8(p1, 0u, s);
-    const half2_t h = __builtin_bit_cast(half2_t, s);
-    const half2_t k = {__builtin_bit_cast(half_t, (uint16_t)0x1eee), __builtin_bit_cast(half_t, (uint16_t)0x1eee)};
-    const half2_t b = {__builtin_bit_cast(half_t, (uint16_t)0xc931), __builtin_bit_cast(half_t, (uint16_t)0xc931)};
-    return __builtin_elementwise_fma(h, k, b);
-}
-
-// The fp16 pair (1024 + bytesum) of two hashes, before the codebook's affine map: the decode
+// The fp16 pair h = (1024 + bytesum) of two hashes, before the codebook's affine map
+// w = fma_fp16(h, 0x1eee, 0xc931) (the bit-exact MUL1 decode; dequant.hip applies it): the decode
 // GEMV multiplies these by the activations and applies w = 0x1eee * h + 0xc931 once per column
 // (sum_k x_k w_k = 0x1eee * sum_k x_k h_k + 0xc931 * sum_k x_k).
 __device__ __forceinline__ half2_t mul1_hpair(uint32_t p0, uint32_t p1)
@@ -71,12 +60,6 @@ __device__ __forceinline__ half2_t mul1_hpair(uint32_t p0, uint32_t p1)
 
 constexpr float MUL1_K_INV = 0.00676727294921875f;   // fp16 0x1eee
 constexpr float MUL1_K_BIAS = -10.3828125f;          // fp16 0xc931
-
-__device__ __forceinline__ half_t mul1_one(uint32_t state)
-{
-    const half2_t w = mul1_pair(mul1_hash<false>(state), 0u);
-    return w.x;
-}
 
 __device__ __forceinline__ float dot2(half2_t a, half2_t b, float c)
 {
@@ -131,14 +114,8 @@ __device__ __forceinline__ uint32_t lane_hash(const LaneWords<K>& w)
     }
 }
 
-// Decoded weight pair of lane-local positions (J, J+1) (J even): same column, k and k+1.
-template <int K, int J>
-__device__ __forceinline__ half2_t lane_pair(const LaneWords<K>& w)
-{
-    return mul1_pair(lane_hash<K, J>(w), lane_hash<K, J + 1>(w));
-}
-
-// The (1024 + bytesum) pair of the same positions (see mul1_hpair).
+// The (1024 + bytesum) pair of lane-local positions (J, J+1) (J even): same column, k and k+1 (see
+// mul1_hpair).
 template <int K, int J>
 __device__ __forceinline__ half2_t lane_hpair(const LaneWords<K>& w)
 {

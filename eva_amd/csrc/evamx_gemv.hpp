@@ -196,7 +196,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t weight_rsrc(const uint32_t* ba
 template <int K>
 __device__ __forceinline__ void load_slice(LaneWords<K>& w, __amdgpu_buffer_rsrc_t rsrc, uint32_t soff, uint32_t lane_off)
 {
-    if constexpr (K == 2) {
+    if constexpr (K == 1) {
+        w.b[1] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, lane_off, soff, BUF_NT);
+    } else if constexpr (K == 2) {
         const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, lane_off, soff, BUF_NT));
         w.b[1] = v.x; w.b[2] = v.y;
     } else if constexpr (K == 3) {

@@ -22,7 +22,7 @@ void launch_fill_i32(int* p, int n, int v, hipStream_t stream);
 // EVAMX_OK, or EVAMX_ELAUNCH with the message set if the last launch failed
 int launched(const char* what);
 
-int launch_dequant(const void* trellis, int in, int out, int k2, void* w, bool scalar, hipStream_t stream);
+int launch_dequant(const void* trellis, int in, int out, int k2, void* w, hipStream_t stream);
 
 }  // namespace evamx
 

@@ -566,3 +566,23 @@ def test_moe_out_of_range_expert_sets_flag(dev):
     rw2[0, 1] = 0                                                  # the flagged slot is dropped
     ref = coop.moe_routed(x, np.where(sel < E, sel, 0), rw2, experts, 0.0)
     assert rel_err_rows(out.cpu().numpy(), ref) < TOL
+
+
+@pytest.mark.parametrize("K", [1, 1.5, 2, 2.5, 3, 3.5, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("shape", [(16, 16), (48, 144), (16, 112), (80, 128)])
+def test_dequant_partial_groups(dev, K, shape):
+    """One k-slice or a few, column counts short of a wave's 8 tiles, every rate: bit-exact, and nothing
+    outside the output is written (the tensor behind it is a larger, pre-filled one)."""
+    ops = _ops()
+    n_in, n_out = shape
+    rng = np.random.default_rng(int(10 * K) + n_out)
+    tr = synth.projection(rng, n_in, n_out, K)[0]
+    w = ops.exl3_dequant(to_dev(tr, dev), K)
+    ref = exl3.dequant(tr, K)
+    assert np.array_equal(w.cpu().numpy().view(np.uint16), ref.view(np.uint16))
+    buf = torch.full((w.numel() + 66,), 7.0, dtype=torch.float16, device=dev)
+    rc = ops.lib().evamx_exl3_dequant(ops.ptr(to_dev(tr, dev)), n_in, n_out, float(K), buf.data_ptr() + 2 * 33, ops.stream_handle(w.device))
+    assert rc == 0
+    got = buf.cpu().numpy()
+    assert np.array_equal(got[33:33 + w.numel()].view(np.uint16), ref.reshape(-1).view(np.uint16))
+    assert (got[:33] == 7.0).all() and (got[33 + w.numel():] == 7.0).all()
