@@ -315,37 +315,6 @@ struct GlobalRows {
     int sums_stride;        // chunks per row
 };
 
-// Activation source of gemv_wave: the 8 fp16 pairs (x[16kt + 2i], x[16kt + 2i + 1]) of row m
-// at k-slice kt. XScalar reads rows of global memory through wave-uniform addresses (scalar
-// loads into SGPRs); XLds reads rows the wave staged in LDS itself (one uniform-address
-// ds_read_b128 pair, a broadcast).
-template <int TM>
-struct XScalar {
-    const half2_t* A;
-    uint32_t aoff[TM];      // row m starts at A + 4 * aoff[m] (aoff in 16-byte units)
-    __device__ __forceinline__ void load(int m, int kt, half2_t (&d)[8]) const
-    {
-        const half2_t* xp = A + ((size_t)aoff[m] * 4 + (size_t)kt * 8);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) d[i] = xp[i];
-    }
-};
-
-// The rows are written and read as uint32_t words (one type, so that no alias rule separates
-// the wave's stores from its loads); rows and slices are 32-byte aligned, so the eight words of
-// a slice merge into wide LDS reads.
-struct XLds {
-    const uint32_t* base;   // LDS: row m at base + m * row_words, k-slice kt at word 8 * (kt - kt0)
-    int row_words;
-    int kt0;
-    __device__ __forceinline__ void load(int m, int kt, half2_t (&d)[8]) const
-    {
-        const uint32_t* xp = (const uint32_t*)__builtin_assume_aligned(base + m * row_words + 8 * (kt - kt0), 32);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) d[i] = __builtin_bit_cast(half2_t, xp[i]);
-    }
-};
-
 // Orders a wave's LDS writes before its later LDS reads of other lanes' data (and its reads
 // before later overwrites): LDS instructions of one wave execute in order, the fence keeps the
 // compiler from moving them across.
@@ -364,111 +333,6 @@ struct NoPrologue {
     __device__ __forceinline__ void issue() {}
     __device__ __forceinline__ void finish() {}
 };
-
-// ---------------------------------------------------------------------------------------------
-// Decode GEMV over one wave's k-range [kt0, kt1): acc[m][h] += sum_k X[m][k] * h_k,
-// h_k = 1024 + bytesum of the weight at (k, col(lane, h)) (see mul1_hpair). The caller zeroes
-// acc. `prologue.issue()` runs just before the weight prefetch ring is issued and
-// `prologue.finish()` once it is in flight (the rotated-input path loads its activation words
-// first and stages its rows in LDS behind the latency of the first weight loads).
-
-// Weight prefetch depth (k-slices in flight per wave). Four slices (4 KiB per wave at 4 bpw)
-// measured best for every chunk width once the waves of a SIMD progress together (depths 4..10
-// at 1 and 2 rows: 4 and 5 the fastest, 10 4% slower).
-template <int TM>
-constexpr int prefetch_depth() { return 4; }
-
-template <int K2, int TM, int PF = prefetch_depth<TM>(), typename XS, typename Pro>
-__device__ __forceinline__ void gemv_wave(const uint32_t* __restrict__ trellis, int nt_n, int cg, int kt0, int kt1,
-                                          const XS& xs, int tm, float (&acc)[TM][2], Pro& prologue)
-{
-    using R = Rate<K2>;
-    constexpr int K = R::K;
-    constexpr int TW = R::TW;
-    const int lane = threadIdx.x & 63;
-    // the k-range is wave-uniform: keep it (and all index math below) in scalar registers
-    kt0 = __builtin_amdgcn_readfirstlane(kt0);
-    kt1 = __builtin_amdgcn_readfirstlane(kt1);
-    // byte offsets: slices are nt_n tiles apart, the wave's 8 tiles start at tile 8*cg; a
-    // projection is at most 7168 x 7168 x 8 bits, far below the 2 GiB buffer range
-    const uint32_t slice = __builtin_amdgcn_readfirstlane(4u * (uint32_t)(nt_n * TW));
-    const uint32_t cbase = __builtin_amdgcn_readfirstlane(4u * (uint32_t)(cg * 8 * TW));
-    const __amdgpu_buffer_rsrc_t rsrc = weight_rsrc(trellis);
-    uint32_t lane_off, sh;
-    lane_offsets<K2>(lane, lane_off, sh);
-
-    // Prefetch ring: the row PF slices ahead, clamped to the wave's last row so that the steady
-    // state needs no branch and never reads outside the matrix (the clamped reloads hit cache).
-    prologue.issue();
-    LaneWords<K> ring[PF];
-    const int last = kt1 - 1;
-#pragma unroll
-    for (int d = 0; d < PF; ++d) load_slice<K>(ring[d], rsrc, cbase + (uint32_t)min(kt0 + d, last) * slice, lane_off);
-    // keep the prologue's work (and its waits for its own loads) after the ring is issued
-    if constexpr (Pro::kWork) __builtin_amdgcn_sched_barrier(0);
-    prologue.finish();
-
-    // Narrow chunks load the next slice's activations one step ahead, so their latency hides
-    // behind a decode instead of stalling every step.
-    constexpr bool XPF = TM <= 2;
-    half2_t xa[TM][8];
-    auto load_x = [&](half2_t (&dst)[TM][8], int kt) {
-#pragma unroll
-        for (int m = 0; m < TM; ++m)
-            if (m < tm) xs.load(m, kt, dst[m]);
-    };
-    if constexpr (XPF) load_x(xa, kt0);
-
-    // Decode the slot, then refill the same registers with the slice PF ahead (issuing the load
-    // before the decode would keep two copies of the slot live and make the compiler rotate
-    // registers through moves that wait for every load in flight), then the dot products.
-    auto step = [&](int kt, LaneWords<K>& w) {
-        half2_t xn[TM][8];
-        if constexpr (XPF) load_x(xn, min(kt + 1, last));
-        half2_t wp[16];
-        decode_slice<K2>(w, sh, wp);
-        load_slice<K>(w, rsrc, cbase + (uint32_t)min(kt + PF, last) * slice, lane_off);
-#pragma unroll
-        for (int m = 0; m < TM; ++m) {
-            if (m < tm) {
-                if constexpr (!XPF) xs.load(m, kt, xa[m]);
-                float a0 = acc[m][0], a1 = acc[m][1];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    a0 = dot2(wp[4 * u + 0], xa[m][u], a0);
-                    a0 = dot2(wp[4 * u + 1], xa[m][u + 4], a0);
-                    a1 = dot2(wp[4 * u + 2], xa[m][u], a1);
-                    a1 = dot2(wp[4 * u + 3], xa[m][u + 4], a1);
-                }
-                acc[m][0] = a0;
-                acc[m][1] = a1;
-            }
-            // wide chunks: keep at most four tokens' activations (32 SGPRs) live at a time
-            if constexpr (TM >= 8)
-                if ((m & 3) == 3) __builtin_amdgcn_sched_barrier(0);
-        }
-        if constexpr (XPF) {
-#pragma unroll
-            for (int m = 0; m < TM; ++m)
-#pragma unroll
-                for (int i = 0; i < 8; ++i) xa[m][i] = xn[m][i];
-        }
-        // keep the next step's activation loads out of this one (register pressure)
-        __builtin_amdgcn_sched_barrier(0);
-    };
-
-    const int n_kt = kt1 - kt0;
-    int kt = kt0;
-    for (; kt + PF <= kt1; kt += PF) {
-        progress_priority(kt - kt0, n_kt);
-#pragma unroll
-        for (int d = 0; d < PF; ++d) step(kt + d, ring[d]);
-    }
-    progress_priority(n_kt, n_kt);
-#pragma unroll
-    for (int d = 0; d < PF - 1; ++d)
-        if (kt + d < kt1) step(kt + d, ring[d]);
-}
 
 // ---------------------------------------------------------------------------------------------
 // The same decode GEMV with the products on the matrix cores: v_mfma_f32_4x4x4_16b_f16 runs 16
@@ -621,64 +485,6 @@ __device__ __forceinline__ float strided_sum(const float* sp, int c0, int c1, in
     }
     return xs;
 }
-
-// GEMV for a chunk of tm rows over the 128-element k-chunks [c0, c1) with the smallest
-// template that fits; writes fp32 partials part[slot_of[m] * part_stride + column] =
-// sum_k x_k w_k = 0x1eee * sum_k x_k h_k + 0xc931 * sum_k x_k.
-// Only the row variants up to TMAX are compiled in, so a launch for narrow chunks is not
-// register-allocated for the widest one. A chunk of more than TMAX rows (possible only when
-// given routes repeat an expert within a token) is processed TMAX rows at a time.
-template <int K2, int TMAX>
-__device__ __forceinline__ void gemv_chunk(const uint32_t* trellis, int nt_n, int cg, int c0, int c1,
-                                           const GlobalRows& src, const int* slot_of, int tm, float* part,
-                                           size_t part_stride)
-{
-    const int lane = threadIdx.x & 63;
-    const int col0 = cg * 128 + lane_col(lane, 0), col1 = cg * 128 + lane_col(lane, 1);
-#define EVAMX_RUN(TMV)                                                                          \
-    {                                                                                           \
-        XScalar<TMV> xsrc;                                                                      \
-        xsrc.A = (const half2_t*)src.A;                                                         \
-        _Pragma("unroll") for (int m = 0; m < TMV; ++m)                                         \
-            xsrc.aoff[m] = (uint32_t)__builtin_amdgcn_readfirstlane((m < tr ? so[m] : so[0]) *   \
-                                                                    (int)(src.stride / 8));     \
-        float acc[TMV][2];                                                                      \
-        _Pragma("unroll") for (int m = 0; m < TMV; ++m) acc[m][0] = acc[m][1] = 0.0f;           \
-        NoPrologue none;                                                                        \
-        gemv_wave<K2, TMV>(trellis, nt_n, cg, 8 * c0, 8 * c1, xsrc, tr, acc, none);              \
-        _Pragma("unroll") for (int m = 0; m < TMV; ++m) {                                       \
-            if (m < tr) {                                                                       \
-                const int row = so[m];                                                          \
-                const float xs = strided_sum<4>(src.sums + (size_t)row * src.sums_stride, c0, c1); \
-                float* dst = part + (size_t)row * part_stride;                                  \
-                dst[col0] = mul1_affine(acc[m][0], xs);                                         \
-                dst[col1] = mul1_affine(acc[m][1], xs);                                         \
-            }                                                                                   \
-        }                                                                                       \
-    }
-    for (int r0 = 0; r0 < tm; r0 += TMAX) {
-        const int* so = slot_of + r0;
-        const int tr = tm - r0 < TMAX ? tm - r0 : TMAX;
-        if constexpr (TMAX == 1) EVAMX_RUN(1)
-        else if constexpr (TMAX == 2) {
-            if (tr <= 1) EVAMX_RUN(1)
-            else EVAMX_RUN(2)
-        } else if constexpr (TMAX == 4) {
-            if (tr <= 2) EVAMX_RUN(2)
-            else EVAMX_RUN(4)
-        } else {
-            static_assert(TMAX == 8, "row bounds are 1, 2, 4 or 8");
-            if (tr <= 1) EVAMX_RUN(1)
-            else if (tr <= 2) EVAMX_RUN(2)
-            else if (tr <= 4) EVAMX_RUN(4)
-            else EVAMX_RUN(8)
-        }
-    }
-#undef EVAMX_RUN
-}
-
-// Smallest compiled row bound that covers `rows` rows per chunk (wider chunks loop over it).
-inline int tmax_for(int rows) { return rows <= 1 ? 1 : rows <= 2 ? 2 : rows <= 4 ? 4 : 8; }
 
 // Sum over the wave of one value per lane (order fixed by the butterfly).
 __device__ __forceinline__ float wave_sum(float v)

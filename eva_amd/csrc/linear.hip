@@ -21,17 +21,7 @@
 namespace evamx {
 
 
-__constant__ int k_iota64[64] = {0,  1,  2,  3,  4,  5,  6,  7,  8,  9,  10, 11, 12, 13, 14, 15,
-                                 16, 17, 18, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28, 29, 30, 31,
-                                 32, 33, 34, 35, 36, 37, 38, 39, 40, 41, 42, 43, 44, 45, 46, 47,
-                                 48, 49, 50, 51, 52, 53, 54, 55, 56, 57, 58, 59, 60, 61, 62, 63};
-
 constexpr int LIN_GEMV_ROWS = 16;     // decode GEMV up to this many rows, MFMA tiles beyond
-constexpr int LIN_ROT_ROWS = 2;       // the GEMV rotates its own inputs up to this many rows
-// Weight prefetch depth of the 1-2 row GEMV: its waves stream 8 k-slices each at 2048 x 7168,
-// one wave per SIMD; 3 slices in flight measured best (2: 7.58, 3: 6.84, 4: 6.98,
-// 5: 7.07 us per call; the MoE's longer items keep 4).
-constexpr int LIN_PF = 3;
 
 struct LinParams {
     const half_t* x;
@@ -40,180 +30,11 @@ struct LinParams {
     const half_t* suh;
     const half_t* svh;
     half_t* y;
-    half_t* xr;        // [rows][in]
+    half_t* xr;        // rotated rows as A operands (a_operand_offset), beyond LIN_GEMV_ROWS rows
     float* xsum;       // [rows][in/128]
-    float* part;       // [ks][rows][out]
+    float* part;       // decode path: [quarters of ks][rows][out]; k-range partials: [ks][rows][out]
     unsigned long long* arrive;   // arrival counters of the decode path, one per ARRIVE_STRIDE words
 };
-
-// Rotated inputs of tm rows (rows r0 .. r0 + tm - 1 of x) over the 128-chunks [w0, w1) into
-// the wave's LDS rows (row m at dst + m * LIN_CW * 64 words, chunk w0 + j at word 64 j), with
-// each row's chunk sums added in chunk order; the same operations as lin_rotate_kernel, so the
-// rows are bit-identical to its output. issue() loads the x and suh words before the weight
-// prefetch ring, finish() rotates them once the ring is in flight.
-constexpr int LIN_CW = 4;             // 128-chunks per LDS window
-
-template <int TM>
-struct LinRot {
-    static constexpr bool kWork = true;
-    const LinParams& p;
-    int tm, w0, w1, lane;
-    __amdgpu_buffer_rsrc_t xrs[TM], srs;
-    uint32_t* dst;
-    float (&xs)[TM];
-    uint32_t xv[TM][LIN_CW], sv[LIN_CW];
-
-    __device__ __forceinline__ void issue()
-    {
-        // chunks past the window reload its last one (in bounds, unused): no branches
-#pragma unroll
-        for (int j = 0; j < LIN_CW; ++j)
-            sv[j] = __builtin_amdgcn_raw_buffer_load_b32(srs, 4 * lane, 256 * min(w0 + j, w1 - 1), 0);
-#pragma unroll
-        for (int m = 0; m < TM; ++m)
-#pragma unroll
-            for (int j = 0; j < LIN_CW; ++j)
-                xv[m][j] = __builtin_amdgcn_raw_buffer_load_b32(xrs[m], 4 * lane, 256 * min(w0 + j, w1 - 1), 0);
-    }
-    __device__ __forceinline__ void finish()
-    {
-#pragma unroll
-        for (int m = 0; m < TM; ++m) {
-            if (m >= tm) continue;
-#pragma unroll
-            for (int j = 0; j < LIN_CW; ++j) {
-                if (w0 + j < w1) {
-                    const half2_t xx = __builtin_bit_cast(half2_t, xv[m][j]);
-                    const half2_t su = __builtin_bit_cast(half2_t, sv[j]);
-                    float v0 = h2f(f2h(h2f(xx.x) * h2f(su.x)));      // fp16 product
-                    float v1 = h2f(f2h(h2f(xx.y) * h2f(su.y)));
-                    had128_pair(v0, v1, lane);
-                    const half2_t r = {f2h(v0), f2h(v1)};
-                    dst[m * LIN_CW * 64 + j * 64 + lane] = __builtin_bit_cast(uint32_t, r);
-                    xs[m] += wave_sum(h2f(r.x) + h2f(r.y));
-                }
-            }
-        }
-        wave_lds_fence();
-    }
-};
-
-template <int K2, int TM>
-__device__ __forceinline__ void lin_rows(const LinParams& p, int r0, int tm, int cg, int ks, int c0, int c1, uint32_t* lds)
-{
-    const int lane = threadIdx.x & 63;
-    __amdgpu_buffer_rsrc_t xrs[TM];
-#pragma unroll
-    for (int m = 0; m < TM; ++m) xrs[m] = weight_rsrc((const uint32_t*)(p.x + (size_t)(r0 + (m < tm ? m : 0)) * p.in));
-    const __amdgpu_buffer_rsrc_t srs = weight_rsrc((const uint32_t*)p.suh);
-    float acc[TM][2], xs[TM];
-#pragma unroll
-    for (int m = 0; m < TM; ++m) acc[m][0] = acc[m][1] = xs[m] = 0.0f;
-    auto window = [&](int w0, int w1) {
-        const XLds src{lds, LIN_CW * 64, 8 * w0};
-        LinRot<TM> stage{p, tm, w0, w1, lane, {}, srs, lds, xs};
-#pragma unroll
-        for (int m = 0; m < TM; ++m) stage.xrs[m] = xrs[m];
-        gemv_wave<K2, TM, LIN_PF>(p.trellis, p.out / 16, cg, 8 * w0, 8 * w1, src, tm, acc, stage);
-    };
-    if (c1 - c0 <= LIN_CW) {
-        window(c0, c1);
-    } else {
-        for (int w0 = c0; w0 < c1; w0 += LIN_CW) {
-            window(w0, min(c1, w0 + LIN_CW));
-            wave_lds_fence();           // this window's reads before the next window's writes
-        }
-    }
-    const int col0 = cg * 128 + lane_col(lane, 0), col1 = cg * 128 + lane_col(lane, 1);
-#pragma unroll
-    for (int m = 0; m < TM; ++m) {
-        if (m < tm) {
-            float* dst = p.part + ((size_t)ks * p.rows + r0 + m) * p.out;
-            store_wt(dst + col0, mul1_affine(acc[m][0], xs[m]));
-            store_wt(dst + col1, mul1_affine(acc[m][1], xs[m]));
-        }
-    }
-}
-
-template <int K2, int TM>
-__device__ __forceinline__ void lin_item(const LinParams& p, int cg, int ks, int c0, int c1, uint32_t* lds)
-{
-    if constexpr (TM == 1) lin_rows<K2, 1>(p, 0, 1, cg, ks, c0, c1, lds);
-    else lin_rows<K2, 2>(p, 0, p.rows, cg, ks, c0, c1, lds);
-}
-
-// Partials of 16 splits for the lane's two columns (byte offsets vo and vo + 32 in rs, splits sb
-// bytes apart from split q0 on), the loads all issued before the adds; splits from `valid` on are
-// loaded clamped and not added. POL LD_SC1: the loads read the memory side, where the other
-// workgroups' write-through stores went; buffer loads take the split offsets in scalar registers,
-// so no vector instruction computes an address.
-
-template <bool FULL, int POL>
-__device__ __forceinline__ void lin_sum16(__amdgpu_buffer_rsrc_t rs, uint32_t vo, uint32_t sb, int q0, int valid,
-                                          float& v0, float& v1)
-{
-    float t0[16], t1[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const uint32_t so = sb * (uint32_t)(q0 + (FULL ? i : min(i, valid - 1)));
-        t0[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, vo, so, POL));
-        t1[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, vo + 32, so, POL));
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-        if (FULL || i < valid) {
-            v0 += t0[i];
-            v1 += t1[i];
-        }
-}
-
-// Output epilogue of row m of a column group: the row's k-split partials summed in split order
-// (one memory round trip per 16 splits), C to fp16, Hadamard, fp16 svh product. POL: LD_SC1 in
-// the launch that wrote the partials (run by the group's last workgroup after its arrival, where
-// every instruction is on the call's critical path), 0 in a launch of its own.
-template <int POL>
-__device__ __forceinline__ void lin_epilogue_row(const LinParams& p, int cg, int m, const float (&sv)[2])
-{
-    const int lane = threadIdx.x & 63;
-    const __amdgpu_buffer_rsrc_t rs = weight_rsrc((const uint32_t*)p.part);
-    const uint32_t vo = 4u * (uint32_t)(m * p.out + cg * 128 + lane_col(lane, 0));   // column 1: + 32 bytes
-    const uint32_t sb = 4u * (uint32_t)(p.rows * p.out);
-    float v0 = 0.0f, v1 = 0.0f;
-    for (int q0 = 0; q0 < p.ks; q0 += 16) {
-        if (q0 + 16 <= p.ks) lin_sum16<true, POL>(rs, vo, sb, q0, 16, v0, v1);
-        else lin_sum16<false, POL>(rs, vo, sb, q0, p.ks - q0, v0, v1);
-    }
-    v0 = h2f(f2h(v0));                  // C in fp16
-    v1 = h2f(f2h(v1));
-    had128_lane(v0, v1, lane);
-    half_t* y = p.y + (size_t)m * p.out + cg * 128 + lane_col(lane, 0);
-    y[0] = f2h(h2f(f2h(v0)) * sv[0]);
-    y[8] = f2h(h2f(f2h(v1)) * sv[1]);
-}
-
-// After a workgroup's waves stored their partials: wait until every store is acknowledged, arrive
-// at the column group's counter, and run the epilogue if last (the stores of every workgroup of
-// the group then precede the loads). One row: wave 0 arrives and runs the epilogue alone, with no
-// second barrier; two: the arrival is shared through LDS and wave m runs row m.
-template <int TM>
-__device__ __forceinline__ void lin_arrive(const LinParams& p, int cg, int n, const float (&sv)[2])
-{
-    unsigned long long* word = p.arrive + (size_t)cg * ARRIVE_STRIDE;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if constexpr (TM == 1) {
-        if (wave != 0) return;
-        int l = 0;
-        if (threadIdx.x == 0) l = arrive_last(word, (unsigned)n);
-        if (__builtin_amdgcn_readfirstlane(l)) lin_epilogue_row<LD_SC1>(p, cg, 0, sv);
-    } else {
-        __shared__ int last;
-        if (threadIdx.x == 0) last = arrive_last(word, (unsigned)n);
-        __syncthreads();
-        if (last && wave < p.rows) lin_epilogue_row<LD_SC1>(p, cg, wave, sv);
-    }
-}
 
 // The lane's two svh values, loaded at the start of the launch (the epilogue needs them only in
 // the last workgroup, but then without waiting for them).
@@ -224,101 +45,331 @@ __device__ __forceinline__ void lin_load_sv(const LinParams& p, int cg, float (&
     sv[1] = h2f(p.svh[cg * 128 + lane_col(lane, 1)]);
 }
 
-// Decode path: one workgroup of four waves per (128 output columns, quarter q of the k-splits),
-// wave w taking split 4q + w (waves past the last split only arrive); each row's reduction order
-// depends only on in/out, never on how many rows share the call. One kernel per rate (the host
-// picks it). TM (1 or 2) rows: inputs rotated in the wave.
-template <int K2, int TM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void lin_gemv_kernel(LinParams p)
+// ---------------------------------------------------------------------------------------------
+// Up to LIN_GEMV_ROWS rows: one launch. A workgroup of eight waves takes 128 output columns and four of
+// the ks k-splits, two waves a split with 64 columns each (two waves a SIMD hide each other's latency).
+// The rows are rotated over the split's k-range into LDS while the first weights are in flight; a wave multiplies the decoded weights, as the B operands they are, by the rows as
+// one 16-row A operand; a further operand of ones gives the rows' sums for the codebook map. So one row
+// and sixteen take the same instructions, and a row's bits do not depend on how many share the call. The
+// four splits' results are added in LDS in order; the quarters meet through memory, and the last
+// workgroup to arrive at the column group's counter adds them in order and runs the output epilogue.
+// Bound by latency: the launch, the first weights, the arrival. (Before: v_dot2 per row and two rows'
+// passes from registers, from three rows on a rotation and an epilogue launch around it. 2048 -> 7168 at 4
+// bpw in a graph, us per call: 1 row 7.6 -> 7.4, 2 rows 9.3 -> 8.6, 8 rows 22.5 -> 9.7, 16 rows 36.6 -> 12.4.)
+
+// 128-chunks of rotated rows in LDS at a time, and words of a row there (padded, so that the 16 rows an
+// operand reads lie in different banks). One row: each wave rotates it for itself; more: the two waves of
+// a split rotate half the rows each.
+template <int TM>
+struct LinStage {
+    static constexpr int CW = TM == 1 ? 4 : 2;
+    static constexpr int ROW = CW * 64 + 4;
+    static constexpr int WORDS = TM == 1 ? ROW : TM * ROW;
+};
+
+// fp16(H128(fp16(x * suh))) of the call's rows over the 128-chunks [w0, w1) into LDS. issue() loads ahead
+// of the weight prefetch, finish() rotates behind it. One row: a chunk on the whole wave; more: 16 lanes
+// a chunk, four (row, chunk) pairs at a time. The same bits either way.
+template <int TM>
+struct LinRot;
+
+template <>
+struct LinRot<1> {
+    uint32_t xv[4], sv[4];
+    __device__ __forceinline__ void issue(const LinParams& p, int w0, int w1, int)
+    {
+        const int lane = threadIdx.x & 63;
+        const __amdgpu_buffer_rsrc_t xrs = weight_rsrc((const uint32_t*)p.x), srs = weight_rsrc((const uint32_t*)p.suh);
+        // chunks past the window reload its last one (in bounds, unused): no branches
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t off = 256u * (uint32_t)min(w0 + j, w1 - 1);
+            sv[j] = __builtin_amdgcn_raw_buffer_load_b32(srs, 4 * lane, off, 0);
+            xv[j] = __builtin_amdgcn_raw_buffer_load_b32(xrs, 4 * lane, off, 0);
+        }
+    }
+    template <int HV>
+    __device__ __forceinline__ void finish(const LinParams&, int w0, int w1, int, uint32_t* dst)
+    {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (w0 + j < w1) {
+                const half2_t xx = __builtin_bit_cast(half2_t, xv[j]), su = __builtin_bit_cast(half2_t, sv[j]);
+                float v0 = h2f(f2h(h2f(xx.x) * h2f(su.x)));      // fp16 product
+                float v1 = h2f(f2h(h2f(xx.y) * h2f(su.y)));
+                had128_pair(v0, v1, lane);
+                const half2_t r = {f2h(v0), f2h(v1)};
+                dst[64 * j + lane] = __builtin_bit_cast(uint32_t, r);
+            }
+        }
+    }
+};
+
+template <>
+struct LinRot<16> {
+    u32x4w xv[4], sv[4];
+    __device__ __forceinline__ void load(const LinParams& p, int w0, int w1, int b)
+    {
+        const int lane = threadIdx.x & 63, nw = w1 - w0, n = p.rows * nw;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int it = min(b + 4 * i + (lane >> 4), n - 1), m = it / nw, c = w0 + it % nw;
+            const size_t k = 128 * c + 8 * oct_piece(lane);
+            xv[i] = *(const __attribute__((address_space(1))) u32x4w*)(p.x + (size_t)m * p.in + k);
+            sv[i] = *(const __attribute__((address_space(1))) u32x4w*)(p.suh + k);
+        }
+    }
+    __device__ __forceinline__ void issue(const LinParams& p, int w0, int w1, int half) { load(p, w0, w1, 16 * half); }
+    template <int HV>
+    __device__ __forceinline__ void finish(const LinParams& p, int w0, int w1, int half, uint32_t* dst)
+    {
+        const int lane = threadIdx.x & 63, nw = w1 - w0, n = p.rows * nw;
+        for (int b = 16 * half; b < n; b += 16 * HV) {
+            if (b >= 16 * HV) load(p, w0, w1, b);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int it = b + 4 * i + (lane >> 4);
+                if (b + 4 * i >= n) break;
+                const uint32_t xu[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w}, su[4] = {sv[i].x, sv[i].y, sv[i].z, sv[i].w};
+                float x[8], h[8];
+                oct_halves(xu, x);
+                oct_halves(su, h);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = h2f(f2h(x[e] * h[e]));       // fp16 product
+                had128_oct(x, lane);
+                u32x4 r;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) r[e] = __builtin_bit_cast(uint32_t, half2_t{f2h(x[2 * e]), f2h(x[2 * e + 1])});
+                if (it < n) *(u32x4*)(dst + (it / nw) * LinStage<16>::ROW + 64 * (it % nw) + 4 * oct_piece(lane)) = r;
+            }
+        }
+    }
+};
+
+// The wave's share of the columns (128 / HV from 128 / HV * half on) over its split's k-range [c0, c1) (128-chunks, none for
+// a wave past the splits): acc[nb][r] = sum_k x_k h_k, ones[r] = sum_k x_k for row 4 g + r and column
+// 128 / HV * half + mfma_col(lane, nb). Every wave of the workgroup runs `windows` windows of CW chunks.
+template <int K2, int TM, int HV>
+__device__ __forceinline__ void lin_gemv_range(const LinParams& p, int cg, int half, int c0, int c1, int windows, uint32_t* lds,
+                                               f32x4_t (&acc)[8 / HV], f32x4_t& ones)
 {
-    __shared__ uint32_t xl[4][TM * LIN_CW * 64];
+    using R = Rate<K2>;
+    constexpr int K = R::K;
+    constexpr int TW = R::TW;
+    constexpr int CW = LinStage<TM>::CW;
+    constexpr int NU = 4 / HV;                            // units (pairs of tiles) a step
+    const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4, nt_n = p.out / 16;
+    const uint32_t slice = __builtin_amdgcn_readfirstlane(4u * (uint32_t)(nt_n * TW));
+    const uint32_t cbase = __builtin_amdgcn_readfirstlane(4u * (uint32_t)((cg * 8 + 2 * NU * half) * TW));
+    const __amdgpu_buffer_rsrc_t rsrc = weight_rsrc(p.trellis);
+    uint32_t lane_off, sh;
+    lane_offsets<K2>(lane & 15, lane_off, sh);
+    lane_off += (uint32_t)g * slice;
+    // rows past the call's read row 0 (their results are dropped)
+    const uint32_t* xrow = lds + (m16 < p.rows ? m16 : 0) * LinStage<TM>::ROW + 8 * g;
+    const half_t o1 = (half_t)1.0f;
+    const half8_t bones = {o1, o1, o1, o1, o1, o1, o1, o1};
+#pragma unroll
+    for (int nb = 0; nb < 2 * NU; ++nb) acc[nb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    ones = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < windows; ++i) {
+        const int w0 = c0 + i * CW, w1 = min(c1, w0 + CW), steps = 2 * (w1 - w0);
+        const uint32_t wbase = cbase + (uint32_t)(8 * w0) * slice;
+        const bool work = w0 < w1;                        // wave-uniform
+        LaneWords<K> ring[HV][NU];                        // HV steps
+        auto load_w = [&](LaneWords<K>& w, int t, int j) {
+            load_slice<K>(w, rsrc, wbase + (uint32_t)(4 * min(t, steps - 1)) * slice + (uint32_t)(8 * j * TW), lane_off);
+        };
+        if (work) {
+            LinRot<TM> rot;
+            rot.issue(p, w0, w1, half);
+#pragma unroll
+            for (int t = 0; t < HV; ++t)
+#pragma unroll
+                for (int j = 0; j < NU; ++j) load_w(ring[t][j], t, j);
+            __builtin_amdgcn_sched_barrier(0);
+            rot.template finish<HV>(p, w0, w1, half, lds);
+        }
+        if constexpr (TM == 1) wave_lds_fence();
+        else __syncthreads();
+        auto step = [&](int t, LaneWords<K> (&w)[NU]) {
+            const half8_t a0 = __builtin_bit_cast(half8_t, *(const u32x4_t*)(xrow + 32 * t));
+            const half8_t a1 = __builtin_bit_cast(half8_t, *(const u32x4_t*)(xrow + 32 * t + 4));
+            ones = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, bones, ones, 0, 0, 0);
+            ones = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, bones, ones, 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < NU; ++j) {
+                half2_t wp[16];
+                decode_slice<K2>(w[j], sh, wp);
+                load_w(w[j], t + HV, j);
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    acc[2 * j + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, mfma_b(wp, c, 0), acc[2 * j + c], 0, 0, 0);
+                    acc[2 * j + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, mfma_b(wp, c, 1), acc[2 * j + c], 0, 0, 0);
+                }
+            }
+        };
+        if (work)
+            for (int t = 0; t < steps; t += 2) {
+                step(t, ring[0]);
+                step(t + 1, ring[HV - 1]);
+            }
+        // this window's reads before the next window's writes (or the results)
+        if constexpr (TM == 1) wave_lds_fence();
+        else __syncthreads();
+    }
+}
+
+// Output epilogue of a row's 128 columns (the lane's two), their codebook map applied: C in fp16,
+// Hadamard, fp16 svh product.
+__device__ __forceinline__ void lin_finish_row(const LinParams& p, int row, int cg, float v0, float v1, const float (&sv)[2])
+{
+    const int lane = threadIdx.x & 63;
+    v0 = h2f(f2h(v0));
+    v1 = h2f(f2h(v1));
+    had128_lane(v0, v1, lane);
+    half_t* y = p.y + (size_t)row * p.out + cg * 128 + lane_col(lane, 0);
+    y[0] = f2h(h2f(f2h(v0)) * sv[0]);
+    y[8] = f2h(h2f(f2h(v1)) * sv[1]);
+}
+
+// The rows r0, r0 + d, .. (NR of them at most, below p.rows) of a column group: the nq quarters' partials
+// added in order, read from the memory side, where the other workgroups' write-through stores went; the
+// loads of a batch of quarters of every row are issued before any add. Buffer loads take the quarters'
+// offsets in scalar registers.
+template <int NR, int QB>
+__device__ __forceinline__ void lin_last_rows(const LinParams& p, int cg, int r0, int d, int nq, const float (&sv)[2])
+{
+    const int lane = threadIdx.x & 63;
+    const __amdgpu_buffer_rsrc_t rs = weight_rsrc((const uint32_t*)p.part);
+    const uint32_t vo = 4u * (uint32_t)(cg * 128 + lane_col(lane, 0));           // column 1: + 32 bytes
+    float v[NR][2];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) v[i][0] = v[i][1] = 0.0f;
+    for (int q0 = 0; q0 < nq; q0 += QB) {
+        float t[NR][QB][2];
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+#pragma unroll
+            for (int q = 0; q < QB; ++q) {
+                const uint32_t so = 4u * (uint32_t)p.out * (uint32_t)(min(q0 + q, nq - 1) * p.rows + min(r0 + i * d, p.rows - 1));
+                t[i][q][0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, vo, so, LD_SC1));
+                t[i][q][1] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, vo + 32, so, LD_SC1));
+            }
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+#pragma unroll
+            for (int q = 0; q < QB; ++q)
+                if (q0 + q < nq) {
+                    v[i][0] += t[i][q][0];
+                    v[i][1] += t[i][q][1];
+                }
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+        if (r0 + i * d < p.rows) lin_finish_row(p, r0 + i * d, cg, v[i][0], v[i][1], sv);
+}
+
+// One row: every quarter in flight up to 16 (a second round trip cost 0.3 us at 10 quarters, clamped loads
+// 0.4 us at 4).
+__device__ __forceinline__ void lin_last_one(const LinParams& p, int cg, int row, int nq, const float (&sv)[2])
+{
+    if (nq <= 4) lin_last_rows<1, 4>(p, cg, row, 1, nq, sv);
+    else if (nq <= 8) lin_last_rows<1, 8>(p, cg, row, 1, nq, sv);
+    else lin_last_rows<1, 16>(p, cg, row, 1, nq, sv);
+}
+
+// TM: 1, or 16 (2 to LIN_GEMV_ROWS rows).
+template <int K2, int TM, int HV>
+__global__ __launch_bounds__(256 * HV) __attribute__((amdgpu_waves_per_eu(TM == 1 ? 4 : 3))) void lin_gemv_kernel(LinParams p)
+{
+    __shared__ uint32_t lds[TM == 1 ? 4 * HV : 4][LinStage<TM>::WORDS];
+    __shared__ float res1[TM == 1 ? 4 : 1][128];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63, g = lane >> 4;
+    const int split = wave / HV, half = wave % HV;
     const int nq = (p.ks + 3) >> 2;
     const int cg = blockIdx.x / nq, q = blockIdx.x % nq;
-    const int ks = __builtin_amdgcn_readfirstlane(4 * q + (threadIdx.x >> 6));
+    const int ks = 4 * q + split, nv = min(4, p.ks - 4 * q);     // the workgroup's splits
     float sv[2];
     lin_load_sv(p, cg, sv);
-    if (ks < p.ks) {
-        const int nch = p.in / 128;
-        const int c0 = nch * ks / p.ks, c1 = nch * (ks + 1) / p.ks;
-        lin_item<K2, TM>(p, cg, ks, c0, c1, xl[threadIdx.x >> 6]);
-    }
-    lin_arrive<TM>(p, cg, nq, sv);
-}
-
-// 3 to LIN_GEMV_ROWS rows: the rows rotated beforehand (lin_rotate_kernel), read through
-// scalar loads (wider row blocks in LDS would not fit the register budget); one wave per (128
-// output columns, k-split), the output epilogue in a launch of its own (lin_epilogue_kernel). At
-// these row counts the last workgroup of a column group would run many rows' epilogues one after
-// another (16 rows at 2048 x 7168: 38.6 us per call, against 32.1 us with the epilogue launch).
-template <int K2, int TMAX>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void lin_gemv_rows_kernel(LinParams p)
-{
-    const int wid = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const int ncg = p.out / 128;
-    if (wid >= ncg * p.ks) return;
-    const int cg = __builtin_amdgcn_readfirstlane(wid / p.ks), ks = __builtin_amdgcn_readfirstlane(wid % p.ks);
     const int nch = p.in / 128;
-    const int c0 = nch * ks / p.ks, c1 = nch * (ks + 1) / p.ks;
-    gemv_chunk<K2, TMAX>(p.trellis, p.out / 16, cg, c0, c1, GlobalRows{p.xr, (size_t)p.in, p.xsum, nch}, k_iota64,
-                         p.rows, p.part + (size_t)ks * p.rows * p.out, (size_t)p.out);
+    const int c0 = split < nv ? nch * ks / p.ks : 0, c1 = split < nv ? nch * (ks + 1) / p.ks : 0;
+    const int windows = ((nch + p.ks - 1) / p.ks + LinStage<TM>::CW - 1) / LinStage<TM>::CW;
+    f32x4_t acc[8 / HV], ones;
+    lin_gemv_range<K2, TM, HV>(p, cg, half, c0, c1, windows, lds[TM == 1 ? wave : split], acc, ones);
+    auto res = [&](int w) { return TM == 1 ? res1[w] : (float*)lds[w]; };        // split w's results [row][128]
+    if (split < nv) {
+        float* d = res(split) + 128 / HV * half;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 4 * g + r;
+            if (TM == 1 ? lane < 16 && r == 0 : row < p.rows) {
+#pragma unroll
+                for (int nb = 0; nb < 8 / HV; ++nb) d[128 * row + mfma_col(lane, nb)] = mul1_affine(acc[nb][r], ones[r]);
+            }
+        }
+    }
+    __syncthreads();
+    auto sum = [&](int i) {                                      // the splits' result i, in split order
+        float t = res(0)[i];
+        for (int w = 1; w < nv; ++w) t += res(w)[i];
+        return t;
+    };
+    if (nq == 1) {
+        // the only quarter: nothing to meet
+        for (int row = wave; row < p.rows; row += 4 * HV)
+            lin_finish_row(p, row, cg, 0.0f + sum(128 * row + lane_col(lane, 0)), 0.0f + sum(128 * row + lane_col(lane, 1)), sv);
+        return;
+    }
+    // store, wait until every store is acknowledged, arrive, and run the epilogue if last (the stores of
+    // every workgroup of the group then precede the loads); one row: wave 0 alone
+    unsigned long long* word = p.arrive + (size_t)cg * ARRIVE_STRIDE;
+    if constexpr (TM == 1) {
+        if (wave != 0) return;
+        float* dst = p.part + (size_t)q * p.out + cg * 128;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) store_wt(dst + lane_col(lane, h), sum(lane_col(lane, h)));
+        if (wave_arrive_last(word, (unsigned)nq)) lin_last_one(p, cg, 0, nq, sv);
+    } else {
+        __shared__ int last;
+        for (int i = threadIdx.x; i < 128 * p.rows; i += 256 * HV)
+            store_wt(p.part + ((size_t)q * p.rows + (i >> 7)) * p.out + cg * 128 + (i & 127), sum(i));
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (threadIdx.x == 0) last = arrive_last(word, (unsigned)nq);
+        __syncthreads();
+        if (last && wave < p.rows) {
+            if (p.rows <= 4 * HV) lin_last_one(p, cg, wave, nq, sv);
+            else lin_last_rows<4 / HV, 4 * HV>(p, cg, wave, 4 * HV, nq, sv);
+        }
+    }
 }
 
-// One wave per (row, 128 output columns).
-__global__ __launch_bounds__(256) void lin_epilogue_kernel(LinParams p)
-{
-    const int wid = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const int ncg = p.out / 128;
-    if (wid >= ncg * p.rows) return;
-    const int m = wid / ncg, cg = wid % ncg;
-    float sv[2];
-    lin_load_sv(p, cg, sv);
-    lin_epilogue_row<0>(p, cg, m, sv);
-}
-
-// Decode path launches of one rate: up to 2 rows one launch (workgroups per (column group, 4
-// splits)); 3 to 16 rows the GEMV (a wave per (column group, split)) and the epilogue.
+// Decode path launch of one rate: workgroups per (column group, four splits), of eight waves while one
+// workgroup a CU leaves the SIMDs a wave each otherwise, of four beyond (5120 x 5120 at 5 bpw, 400
+// workgroups: one row 11.3 against 12.6 us, 13 rows 16.0 against 20.0; 7168 -> 2048 at 2.5 bpw, 224: one row
+// 7.7 against 7.3, 8 rows 11.0 against 10.1).
 template <int K2>
 void launch_gemv_rate(const LinParams& p, hipStream_t stream)
 {
-    const int ncg = p.out / 128;
-    if (p.rows <= LIN_ROT_ROWS) {
-        const dim3 grid((unsigned)(ncg * ((p.ks + 3) / 4)));
-        if (p.rows == 1) hipLaunchKernelGGL((lin_gemv_kernel<K2, 1>), grid, dim3(256), 0, stream, p);
-        else hipLaunchKernelGGL((lin_gemv_kernel<K2, 2>), grid, dim3(256), 0, stream, p);
-        return;
+    const int blocks = p.out / 128 * ((p.ks + 3) / 4);
+    const dim3 grid((unsigned)blocks);
+    if (blocks <= 256) {
+        if (p.rows == 1) hipLaunchKernelGGL((lin_gemv_kernel<K2, 1, 2>), grid, dim3(512), 0, stream, p);
+        else hipLaunchKernelGGL((lin_gemv_kernel<K2, 16, 2>), grid, dim3(512), 0, stream, p);
+    } else {
+        if (p.rows == 1) hipLaunchKernelGGL((lin_gemv_kernel<K2, 1, 1>), grid, dim3(256), 0, stream, p);
+        else hipLaunchKernelGGL((lin_gemv_kernel<K2, 16, 1>), grid, dim3(256), 0, stream, p);
     }
-    const dim3 grid((unsigned)((ncg * p.ks + 3) / 4));
-    if (p.rows <= 4) hipLaunchKernelGGL((lin_gemv_rows_kernel<K2, 4>), grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((lin_gemv_rows_kernel<K2, 8>), grid, dim3(256), 0, stream, p);
-    hipLaunchKernelGGL(lin_epilogue_kernel, dim3((unsigned)((ncg * p.rows + 3) / 4)), dim3(256), 0, stream, p);
 }
 
 // ---------------------------------------------------------------------------------------------
-// More than LIN_GEMV_ROWS rows (and the rotation of 3 to LIN_GEMV_ROWS rows).
+// More than LIN_GEMV_ROWS rows.
 
 constexpr int LIN_RANGES = 8;         // k-ranges whose sums are added in order
 
-// fp16(H128(fp16(x * suh))) of every (row, 128-chunk) with the chunk's sum: one wave each.
-__global__ __launch_bounds__(256) void lin_rotate_kernel(LinParams p)
-{
-    const int lane = threadIdx.x & 63;
-    const int item = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const int nch = p.in / 128;
-    if (item >= p.rows * nch) return;
-    const int r = item / nch, c = item % nch;
-    const uint32_t xw = ((const uint32_t*)(p.x + (size_t)r * p.in + c * 128))[lane];
-    const uint32_t sw = ((const uint32_t*)(p.suh + c * 128))[lane];
-    const half2_t xx = __builtin_bit_cast(half2_t, xw), su = __builtin_bit_cast(half2_t, sw);
-    float v0 = h2f(f2h(h2f(xx.x) * h2f(su.x)));        // fp16 product
-    float v1 = h2f(f2h(h2f(xx.y) * h2f(su.y)));
-    had128_pair(v0, v1, lane);
-    const half2_t o = {f2h(v0), f2h(v1)};
-    ((uint32_t*)(p.xr + (size_t)r * p.in + c * 128))[lane] = __builtin_bit_cast(uint32_t, o);
-    const float sum = wave_sum(h2f(o.x) + h2f(o.y));
-    if (lane == 0) p.xsum[(size_t)r * nch + c] = sum;
-}
-
-// The same rotations for calls of more than LIN_GEMV_ROWS rows, written as A operands
+// fp16(H128(fp16(x * suh))) of the rows with each 128-chunk's sum, written as A operands
 // (a_operand_offset): one workgroup per (16 rows, 128-chunk), each wave four rows, which meet in LDS and
 // leave as the chunk's 4 KiB. Rows past the call's are zero.
 __global__ __launch_bounds__(256) void lin_rotate16_kernel(LinParams p)
@@ -360,17 +411,10 @@ __device__ __forceinline__ float lin_row_total(const LinParams& p, int row)
     return wave_sum(strided_sum<2>(p.xsum + (size_t)row * nch, threadIdx.x & 63, nch, 64));
 }
 
-// Output epilogue of a row's 128 accumulated columns (the lane's two): codebook map, C in fp16, Hadamard,
-// fp16 svh product.
+// lin_finish_row of a row's accumulated columns: the codebook map first.
 __device__ __forceinline__ void lin_store_row(const LinParams& p, int row, int cg, float v0, float v1, float xs, const float (&sv)[2])
 {
-    const int lane = threadIdx.x & 63;
-    v0 = h2f(f2h(mul1_affine(v0, xs)));
-    v1 = h2f(f2h(mul1_affine(v1, xs)));
-    had128_lane(v0, v1, lane);
-    half_t* y = p.y + (size_t)row * p.out + cg * 128 + lane_col(lane, 0);
-    y[0] = f2h(h2f(f2h(v0)) * sv[0]);
-    y[8] = f2h(h2f(f2h(v1)) * sv[1]);
+    lin_finish_row(p, row, cg, mul1_affine(v0, xs), mul1_affine(v1, xs), sv);
 }
 
 // Calls of more than LIN_GEMV_ROWS rows with too few wide tiles to fill the device: one workgroup per
@@ -621,9 +665,9 @@ int linear_ksplit(int rows, int in, int out)
 }
 
 // Workspace: the column groups' arrival counters (out/128 of them, 128 bytes apart, at offset 0
-// for every row count, so that no other layout overwrites them); from 3 rows the rotated rows
-// [rows][in] fp16 and their 128-chunk sums [rows][in/128]; up to 16 rows the fp32 partials
-// [ks][rows][out].
+// for every row count, so that no other layout overwrites them); beyond LIN_GEMV_ROWS rows the rotated
+// rows in blocks of 16 and their 128-chunk sums [rows][in/128]; the fp32 partials of the decode path's
+// quarters or of the k-ranges.
 static size_t arrive_bytes(int out) { return (size_t)(out / 128) * ARRIVE_STRIDE * 8; }
 
 size_t linear_workspace(int rows, int in, int out, size_t* off_part, size_t* off_sum)
@@ -632,16 +676,24 @@ size_t linear_workspace(int rows, int in, int out, size_t* off_part, size_t* off
     size_t o = al(arrive_bytes(out));
     if (off_sum) *off_sum = 0;
     if (off_part) *off_part = 0;
-    if (rows > LIN_ROT_ROWS) {
-        o = al(o + (size_t)(rows > LIN_GEMV_ROWS ? (rows + 15) & ~15 : rows) * in * 2);
+    const bool decode = rows <= LIN_GEMV_ROWS;
+    if (!decode) {
+        o = al(o + (size_t)((rows + 15) & ~15) * in * 2);
         if (off_sum) *off_sum = o;
         o = al(o + (size_t)rows * (in / 128) * 4);
     }
-    if (rows <= LIN_GEMV_ROWS || linear_kind(rows, in, out) == LIN_SPLIT) {
+    if (decode || linear_kind(rows, in, out) == LIN_SPLIT) {
         if (off_part) *off_part = o;
-        o = al(o + (size_t)linear_ksplit(rows, in, out) * rows * out * 4);
+        const int ks = linear_ksplit(rows, in, out);
+        o = al(o + (size_t)(decode ? (ks + 3) / 4 : ks) * rows * out * 4);
     }
     return o;
+}
+
+// Whether the decode path takes the shape: less than 2 GiB of one partial a split.
+bool linear_decode_fits(int rows, int in, int out)
+{
+    return (size_t)linear_ksplit(rows, in, out) * rows * out * 4 + (size_t)rows * in * 2 + arrive_bytes(out) < ((size_t)1 << 31);
 }
 
 int launch_linear(const void* x, int rows, int in, int out, const void* trellis, const void* suh,
@@ -650,6 +702,7 @@ int launch_linear(const void* x, int rows, int in, int out, const void* trellis,
     LinParams p;
     size_t off_part, off_sum;
     linear_workspace(rows, in, out, &off_part, &off_sum);
+    const int kind_ws = rows > LIN_GEMV_ROWS ? linear_kind(rows, in, out) : -1;
     p.x = (const half_t*)x;
     p.rows = rows; p.in = in; p.out = out; p.k2 = k2;
     p.ks = linear_ksplit(rows, in, out);
@@ -657,19 +710,14 @@ int launch_linear(const void* x, int rows, int in, int out, const void* trellis,
     p.suh = (const half_t*)suh;
     p.svh = (const half_t*)svh;
     p.y = (half_t*)y;
-    const size_t off_xr = (arrive_bytes(out) + 255) & ~(size_t)255;
     p.arrive = (unsigned long long*)ws;
-    p.xr = rows > LIN_ROT_ROWS ? (half_t*)((char*)ws + off_xr) : nullptr;
-    p.xsum = rows > LIN_ROT_ROWS ? (float*)((char*)ws + off_sum) : nullptr;
-    p.part = rows <= LIN_GEMV_ROWS || linear_kind(rows, in, out) == LIN_SPLIT ? (float*)((char*)ws + off_part) : nullptr;
-    if (rows > LIN_GEMV_ROWS) {
+    p.xr = kind_ws >= 0 ? (half_t*)((char*)ws + ((arrive_bytes(out) + 255) & ~(size_t)255)) : nullptr;
+    p.xsum = kind_ws >= 0 ? (float*)((char*)ws + off_sum) : nullptr;
+    p.part = off_part ? (float*)((char*)ws + off_part) : nullptr;
+    // the wide kernel's stores are 16 bytes wide
+    const int kind = kind_ws == LIN_WIDE && ((uintptr_t)y & 15) ? (int)LIN_FULL : kind_ws;
+    if (kind >= 0)
         hipLaunchKernelGGL(lin_rotate16_kernel, dim3((unsigned)((rows + 15) / 16 * (in / 128))), dim3(256), 0, stream, p);
-    } else if (rows > LIN_ROT_ROWS) {
-        const long waves = (long)rows * (in / 128);
-        hipLaunchKernelGGL(lin_rotate_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, p);
-    }
-    int kind = rows > LIN_GEMV_ROWS ? linear_kind(rows, in, out) : -1;
-    if (kind == LIN_WIDE && ((uintptr_t)y & 15)) kind = LIN_FULL;      // its stores are 16 bytes wide
 #define EVAMX_LIN_RATE(K2)                                   \
     case K2:                                                 \
         if (kind >= 0) launch_rows_rate<K2>(p, kind, stream); \

@@ -149,3 +149,22 @@ def test_linear_row_kernels(dev, shape, K, counts):
     buf = torch.zeros(rows * n_out + 1, dtype=torch.float16, device=dev)
     ops.exl3_linear(xd, lin.trellis, lin.suh, lin.svh, K, out=buf[1:].view(rows, n_out))
     assert torch.equal(buf[1:].view(rows, n_out).view(torch.int16), lin.forward(xd).view(torch.int16))
+
+
+@pytest.mark.parametrize("shape,K", [((128, 128), 4), ((512, 256), 2), ((640, 1024), 3.5), ((5120, 5120), 5), ((1280, 40960), 1.5)])
+def test_linear_decode_rows_bit_identical(dev, shape, K):
+    """1 to 16 rows: one k-split quarter and many, workgroups of four and of eight waves, one and several
+    128-chunks a split. Every row has the bits of its one-row call; those are held to the oracle."""
+    n_in, n_out = shape
+    rng = np.random.default_rng(n_in + n_out)
+    tr, suh, svh = synth.projection(rng, n_in, n_out, K, n_in ** -0.5)
+    from eva_amd.linear import build_linear
+    lin = build_linear(to_dev(suh, dev), to_dev(svh, dev), to_dev(tr, dev), device=dev)
+    x = rng.standard_normal((16, n_in)).astype(np.float16)
+    xd = to_dev(x, dev)
+    one = torch.cat([lin.forward(xd[r:r + 1]) for r in range(16)])
+    for rows in (2, 3, 4, 5, 7, 8, 9, 13, 16):
+        assert torch.equal(lin.forward(xd[:rows]).view(torch.int16), one[:rows].view(torch.int16)), rows
+    if n_out <= 5120:
+        ref = coop.exl3_linear(x[:2], tr, suh, svh, K)
+        assert rel_err_rows(one[:2].cpu().numpy().astype(np.float32), ref.astype(np.float32)) < TOL
