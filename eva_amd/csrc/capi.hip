@@ -221,7 +221,7 @@ extern "C" int evamx_exl3_dequant(const void* trellis, int in_features, int out_
 extern "C" size_t evamx_exl3_linear_workspace_bytes(int rows, int in_features, int out_features)
 {
     if (rows < 1 || rows > 65536 || in_features < 128 || out_features < 128) return 0;
-    return linear_workspace(rows, in_features, out_features, nullptr, nullptr);
+    return linear_workspace_upto(rows, in_features, out_features);
 }
 
 extern "C" int evamx_exl3_linear(const void* x_fp16, int rows, int in_features, int out_features, const void* trellis,

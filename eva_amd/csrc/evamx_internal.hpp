@@ -29,6 +29,7 @@ int launch_dequant(const void* trellis, int in, int out, int k2, void* w, hipStr
 namespace evamx {
 
 size_t linear_workspace(int rows, int in, int out, size_t* off_part, size_t* off_sum);
+size_t linear_workspace_upto(int rows, int in, int out);
 bool linear_decode_fits(int rows, int in, int out);
 int launch_linear(const void* x, int rows, int in, int out, const void* trellis, const void* suh,
                   const void* svh, int k2, void* y, void* ws, hipStream_t stream);

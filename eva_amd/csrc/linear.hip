@@ -15,6 +15,8 @@
 // of its own. All add the same k-ranges' sums in the same order. In both paths (up to
 // LIN_GEMV_ROWS rows, and beyond) a row's arithmetic depends on in/out only, not on how many rows
 // share the call.
+#include <algorithm>
+
 #include "evamx_internal.hpp"
 #include "evamx_wide.hpp"
 
@@ -688,6 +690,26 @@ size_t linear_workspace(int rows, int in, int out, size_t* off_part, size_t* off
         o = al(o + (size_t)(decode ? (ks + 3) / 4 : ks) * rows * out * 4);
     }
     return o;
+}
+
+// What a program is told to keep for calls of up to `rows` rows. The k-ranges' partials go only with the
+// row counts between the decode path and the unsplit kernels, so a smaller call can need more than a
+// larger one: the largest need of any row count up to this, so that a workspace made for the largest call
+// (and captured with it) serves the smaller ones too.
+size_t linear_workspace_upto(int rows, int in, int out)
+{
+    size_t n = linear_workspace(rows, in, out, nullptr, nullptr);
+    if (rows <= LIN_GEMV_ROWS) return n;
+    auto most = [&](int r) {
+        const size_t v = linear_workspace(r < rows ? r : rows, in, out, nullptr, nullptr);
+        if (v > n) n = v;
+    };
+    most(LIN_GEMV_ROWS);
+    // the last row count before either unsplit kernel takes over (linear_kind's lines)
+    const long ncg = out / 128, full = 80 + in / 76, wide = 80 + 114688 / in;
+    const long last = std::min((full + ncg - 1) / ncg * LM_ROWS - LM_ROWS, (wide + ncg - 1) / ncg * LW_ROWS - LW_ROWS);
+    if (last > LIN_GEMV_ROWS) most((int)std::min(last, 65536L));
+    return n;
 }
 
 // Whether the decode path takes the shape: less than 2 GiB of one partial a split.

@@ -58,12 +58,13 @@ int evamx_exl3_dequant(const void* trellis, int in_features, int out_features, f
 
 /* ---- single EXL3 linear (fp16 in, fp16 out) ---------------------------------------------- */
 
+/* Bytes that serve calls of up to `rows` rows. */
 size_t evamx_exl3_linear_workspace_bytes(int rows, int in_features, int out_features);
 
 /* y[rows][out] = svh * H(W^T H(x * suh)) with the reference's fp16 rounding points.
  * rows in 1..65536 (up to 16 rows a decode GEMV, beyond it MFMA tiles; within each a row's result
  * does not depend on how many rows share the call); in/out multiples of 128; bits in
- * {1.5,2,2.5,3,3.5,4,5}. All pointers device. Up to 2 rows the call is one launch: the
+ * {1.5,2,2.5,3,3.5,4,5}. All pointers device. Up to 16 rows the call is one launch: the
  * workgroups of each 128-column group meet at an arrival counter kept in the workspace, which may
  * hold anything before its first use (the call then counts with compare-and-swap) and is left at
  * rest by every call, graph replays included. Calls that share a workspace must not overlap. */

@@ -176,3 +176,14 @@ def test_runners_refuse_to_run_without_gpu():
         pytest.skip("a GPU is present")
     with pytest.raises(RuntimeError, match="GPU"):
         CoopRunner3072("cuda:0", topk=6, hidden=256, inter=128, max_rows=4)
+
+
+@pytest.mark.parametrize("n_in,n_out", [(128, 128), (1024, 1024), (1152, 1024), (7168, 896), (7168, 2048), (2048, 7168),
+                                        (5120, 5120), (896, 40960), (65536, 128)])
+def test_linear_workspace_serves_smaller_calls(n_in, n_out):
+    """A workspace made for a larger call serves every smaller one: the bytes never fall with the rows,
+    over the switches between the kernels (some of which keep partials and some do not)."""
+    L = _lib.lib()
+    counts = sorted({*range(1, 70), *(r + d for r in range(64, 4200, 64) for d in (-1, 0, 1)), 8192, 65535, 65536})
+    need = [L.evamx_exl3_linear_workspace_bytes(r, n_in, n_out) for r in counts]
+    assert all(a <= b for a, b in zip(need, need[1:]))
