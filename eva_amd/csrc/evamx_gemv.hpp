@@ -4,9 +4,9 @@
 // one vector load per k-slice and owns output columns 16i+q and 16i+q+8 of the 128-column group
 // for all 16 k of the tile, so the k-loop needs no cross-lane reduction and a wave's 128 columns
 // are exactly one Hadamard chunk. The 16 decoded k of a column pair up as (k, k+1). The MoE
-// decode path multiplies them on the matrix cores (gemv_wave_m4: each lane quad is one
-// v_mfma_f32_4x4x4_16b_f16 block); the single linear's GEMV meets the activation pairs
-// (x[2m], x[2m+1]) in v_dot2_f32_f16 (gemv_wave), both with fp32 accumulation.
+// decode path multiplies them on the matrix cores with fp32 accumulation (gemv_wave_m4: each lane
+// quad is one v_mfma_f32_4x4x4_16b_f16 block). The single linear and the MFMA tiles take the same
+// decode with the lanes 2 tiles across by 4 k-slices down (evamx_mfma.hpp).
 #pragma once
 #include "evamx_device.hpp"
 
@@ -325,17 +325,8 @@ __device__ __forceinline__ void wave_lds_fence()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Work gemv_wave does around issuing its weight prefetch: issue() runs before the first weight
-// loads (loads issued there return first: vector memory loads return in order), finish() once
-// they are in flight.
-struct NoPrologue {
-    static constexpr bool kWork = false;
-    __device__ __forceinline__ void issue() {}
-    __device__ __forceinline__ void finish() {}
-};
-
 // ---------------------------------------------------------------------------------------------
-// The same decode GEMV with the products on the matrix cores: v_mfma_f32_4x4x4_16b_f16 runs 16
+// The decode GEMV's products on the matrix cores: v_mfma_f32_4x4x4_16b_f16 runs 16
 // independent 4x4x4 blocks, block b on lanes 4b..4b+3, and the decode layout's lane quads are
 // exactly such blocks (the four lanes of a quad own four columns of one tile at the same k).
 // Lane 4b + j supplies column j of its block as the B operand (the four k of a k-group from its
@@ -392,8 +383,9 @@ __device__ __forceinline__ half4_t m4_a(const uint32_t (&a)[8], int kg)
 }
 
 // acc[g][c][i] += sum_k X[4g + i][k] * h_k over the wave's k-range [kt0, kt1) for the lane's column
-// c, for tm >= 1 rows; groups g with 4g >= tm are skipped. Same ring, decode and prologue protocol
-// as gemv_wave.
+// c, for tm >= 1 rows; groups g with 4g >= tm are skipped. prologue.issue() runs
+// before the first weight loads (loads issued there return first: vector memory loads return in
+// order), prologue.finish() once they are in flight.
 template <int K2, int NG, int PF = 4, typename Pro>
 __device__ __forceinline__ void gemv_wave_m4(const uint32_t* __restrict__ trellis, int nt_n, int cg, int kt0, int kt1,
                                              const XLds4<NG>& xs, int tm, f32x4v_t (&acc)[NG][2], Pro& prologue)
@@ -415,7 +407,7 @@ __device__ __forceinline__ void gemv_wave_m4(const uint32_t* __restrict__ trelli
     const int last = kt1 - 1;
 #pragma unroll
     for (int d = 0; d < PF; ++d) load_slice<K>(ring[d], rsrc, cbase + (uint32_t)min(kt0 + d, last) * slice, lane_off);
-    if constexpr (Pro::kWork) __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_sched_barrier(0);
     prologue.finish();
 
     // The loop over the k-slices for NA active groups (the groups holding rows), with no branch

@@ -3,12 +3,11 @@
 // Reference: ELinear.forward -> LinearEXL3 (runtime/ds41/exl3_linear.py:97-131), kernel
 // exl3_gemv_kernel.cuh:217-234 (input: fp16 x*suh, Hadamard, fp16), 295-459 (GEMV, fp16 C),
 // 463-490 with hadamard_inner.cuh:93-147 (output Hadamard to fp16, fp16 product with svh).
-// Up to 2 rows, one launch: a k-split decode GEMV whose waves rotate their own input chunks
-// (fp16(H128(fp16(x * suh)))) into LDS while their first weight loads are in flight, writing fp32
-// partials; the workgroup that arrives last at its column group's counter then runs that group's
-// output epilogue (the partials summed in fixed split order, fp16 C, Hadamard, fp16 svh product).
-// 3 to 16 rows, three launches: the input rotation, the same GEMV on the rotated rows, and the
-// same epilogue in a launch of its own.
+// Up to LIN_GEMV_ROWS rows, one launch: a k-split GEMV whose waves rotate their own input chunks
+// (fp16(H128(fp16(x * suh)))) into LDS while their first weight loads are in flight and multiply the
+// decoded weights by the rows as 16-row matrix operands; a workgroup adds its four splits in LDS and
+// writes them as fp32 partials; the workgroup that arrives last at its column group's counter then runs
+// that group's output epilogue (the partials summed in fixed order, fp16 C, Hadamard, fp16 svh product).
 // More rows: the input rotation, written as MFMA operands, then one of three MFMA kernels by size
 // (linear_kind): 256-row workgroups that share each decoded weight (lin_wide_kernel), 64-row
 // workgroups over the whole k range, or over one k-range each with the output epilogue in a launch
@@ -23,7 +22,7 @@
 namespace evamx {
 
 
-constexpr int LIN_GEMV_ROWS = 16;     // decode GEMV up to this many rows, MFMA tiles beyond
+constexpr int LIN_GEMV_ROWS = 16;     // lin_gemv_kernel up to this many rows
 
 struct LinParams {
     const half_t* x;
@@ -50,9 +49,10 @@ __device__ __forceinline__ void lin_load_sv(const LinParams& p, int cg, float (&
 // ---------------------------------------------------------------------------------------------
 // Up to LIN_GEMV_ROWS rows: one launch. A workgroup of eight waves takes 128 output columns and four of
 // the ks k-splits, two waves a split with 64 columns each (two waves a SIMD hide each other's latency).
-// The rows are rotated over the split's k-range into LDS while the first weights are in flight; a wave multiplies the decoded weights, as the B operands they are, by the rows as
-// one 16-row A operand; a further operand of ones gives the rows' sums for the codebook map. So one row
-// and sixteen take the same instructions, and a row's bits do not depend on how many share the call. The
+// The rows are rotated over the split's k-range into LDS while the first weights are in flight; a wave
+// multiplies the decoded weights, as the B operands they are, by the rows as one 16-row A operand; a
+// further operand of ones gives the rows' sums for the codebook map. So one row and sixteen take the same
+// instructions, and a row's bits do not depend on how many share the call. The
 // four splits' results are added in LDS in order; the quarters meet through memory, and the last
 // workgroup to arrive at the column group's counter adds them in order and runs the output epilogue.
 // Bound by latency: the launch, the first weights, the arrival. (Before: v_dot2 per row and two rows'

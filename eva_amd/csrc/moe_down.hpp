@@ -20,7 +20,6 @@ constexpr int DOWN_PF = 3;
 // bounds and unused), finish() stores them.
 template <int TM>
 struct ActStage {
-    static constexpr bool kWork = true;
     int tm, w0, w1, lane;
     __amdgpu_buffer_rsrc_t rs[TM];
     uint32_t* dst;
@@ -75,7 +74,7 @@ __device__ __forceinline__ void down_rows(const MoeParams& p, const uint32_t* tr
 #pragma unroll
     for (int m = 0; m < TM; ++m) {
         if (m < tm) {
-            const float xs = strided_sum<4>(p.actsum + (size_t)so[m] * na, c0, c1);   // chunk order, as gemv_chunk
+            const float xs = strided_sum<4>(p.actsum + (size_t)so[m] * na, c0, c1);   // in chunk order
             float* dst = part + (size_t)so[m] * p.H;
             dst[col0] = mul1_affine(acc[m / 4][0][m % 4], xs);
             dst[col1] = mul1_affine(acc[m / 4][1][m % 4], xs);

@@ -20,7 +20,6 @@ constexpr int DOWN_PAIR_PF = 3;
 // the window copies nothing), then the workgroup meets at a barrier.
 template <int TM>
 struct ActStageGroup {
-    static constexpr bool kWork = true;
     int tm, w0, w1, lane, wave;
     __amdgpu_buffer_rsrc_t rs;                    // the activation rows' base
     const uint32_t (&roff)[TM];                   // byte offset of each row

@@ -24,7 +24,6 @@ constexpr int ROT_CW = 16;            // 128-chunks of rotated input per LDS win
 // (and any further chunks of the window, loading them then).
 template <int TM>
 struct RotStage {
-    static constexpr bool kWork = true;
     const MoeParams& p;
     const int (&so)[TM];
     int tm, w0, w1, row_words, lane;
@@ -96,7 +95,6 @@ constexpr int ROT_WAVES = 4;
 
 template <int TM, int NW = ROT_WAVES, int CW = ROT_CW>
 struct RotStageGroup {
-    static constexpr bool kWork = true;
     static constexpr int NJ = CW / NW;                 // chunks per wave and window
     static_assert(CW % NW == 0, "a window's chunks split evenly over the waves");
     const MoeParams& p;
