@@ -941,8 +941,8 @@ def run_linear(torch, args):
         "step_bytes": int(nbytes), "frac_hbm_step": round(gbps / PEAK_HBM, 4),
         "roofline": {"bound": "hbm", "kernel": "exl3_linear (" + (
                          "1 launch: GEMV with its input rotation, the epilogue in each column group's last workgroup"
-                         if T <= 2 else "3 launches: rotation, GEMV, epilogue" if T <= 16
-                         else "2 launches: rotation, MFMA tiles with their epilogue") + " per call)",
+                         if T <= 16
+                         else "rotation, then MFMA tiles with their epilogue or it in a third launch") + " per call)",
                      "achieved": round(gbps, 1),
                      "peak": PEAK_HBM, "unit": "GB/s", "frac": round(gbps / PEAK_HBM, 4), "traffic": None},
     }
