@@ -37,8 +37,15 @@ class ELinear:
         self._ws = None
 
     def _workspace(self, rows):
-        need = ops.lib().evamx_exl3_linear_workspace_bytes(rows, self.in_features, self.out_features)
-        if self._ws is None or self._ws.numel() < need:
+        """Workspace of a call of ``rows`` rows. Up to GEMV_MAX_ROWS rows the module's own buffer: made
+        once, for GEMV_MAX_ROWS rows, and never replaced, since a captured call goes on using its address
+        (and its arrival counters, which a call leaves at rest for the next). More rows None: the call
+        allocates its own on its stream, so the module holds none of the k-ranges' partials (33 MB for
+        200 rows of 5120 x 5120) and a capture's pool keeps a captured call's as long as the graph."""
+        if rows > GEMV_MAX_ROWS:
+            return None
+        if self._ws is None:
+            need = ops.lib().evamx_exl3_linear_workspace_bytes(GEMV_MAX_ROWS, self.in_features, self.out_features)
             self._ws = torch.empty(need, dtype=torch.uint8, device=self.trellis.device)
         return self._ws
 

@@ -168,3 +168,33 @@ def test_linear_decode_rows_bit_identical(dev, shape, K):
     if n_out <= 5120:
         ref = coop.exl3_linear(x[:2], tr, suh, svh, K)
         assert rel_err_rows(one[:2].cpu().numpy().astype(np.float32), ref.astype(np.float32)) < TOL
+
+
+@pytest.mark.parametrize("rows", [1, 13])
+def test_elinear_graph_after_larger_calls(dev, rows):
+    """A captured call of up to 16 rows keeps a workspace of its own: eager calls of more rows and fresh
+    allocations between its replays change neither its results nor those allocations."""
+    n_in, n_out, K = 1024, 2048, 4
+    rng = np.random.default_rng(5 + rows)
+    tr, suh, svh = synth.projection(rng, n_in, n_out, K, n_in ** -0.5)
+    from eva_amd.linear import build_linear
+    lin = build_linear(to_dev(suh, dev), to_dev(svh, dev), to_dev(tr, dev), device=dev, strict=False)
+    x = to_dev(rng.standard_normal((1024, n_in)).astype(np.float16), dev)
+    xs = x[:rows].clone()
+    want = lin.forward(xs).clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = lin.forward(xs)
+    held = []
+    for more in (17, 200, 1024):
+        big = lin.forward(x[:more]).clone()
+        need = [lin._ws.numel()] + [1 << s for s in range(12, 25)]
+        held += [torch.full((n,), 0x5A, dtype=torch.uint8, device=dev) for n in need]
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+        assert all(bool((t == 0x5A).all()) for t in held)
+        assert torch.equal(lin.forward(x[:more]).view(torch.int16), big.view(torch.int16))
