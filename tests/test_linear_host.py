@@ -44,3 +44,11 @@ def test_larger_calls_keep_no_workspace(monkeypatch):
         lin.forward(torch.zeros(rows, 1024, dtype=torch.float16))
     held = {v.data_ptr() for v in vars(lin).values() if isinstance(v, torch.Tensor)}
     assert not any(ws.data_ptr() in held for rows, ws in calls if rows > GEMV_MAX_ROWS)
+
+
+@pytest.mark.parametrize("n_in,n_out", [(7168, 18432), (4096, 14336), (7168, 12288), (18432, 12288)])
+@pytest.mark.parametrize("rows", [17, 64])
+def test_few_rows_of_a_wide_output_are_split(n_in, n_out, rows):
+    """A call of one 64-row tile keeps the partials of eight k-ranges however many column groups it has:
+    it does not go to the 256-row workgroups, which would be all but empty."""
+    assert _lib.lib().evamx_exl3_linear_workspace_bytes(rows, n_in, n_out) >= 8 * rows * n_out * 4
