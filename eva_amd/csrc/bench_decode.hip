@@ -27,11 +27,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void b
     const half4_t x = {(half_t)0.5f, (half_t)-0.25f, (half_t)0.125f, (half_t)1.0f};
     for (int it = 0; it < iters; ++it) {
         half2_t wp[16];
-        decode_slice<K2>(w, sh, wp);
+        decode_slice<K2, true>(w, sh, wp);
+        mfma_begin();
 #pragma unroll
         for (int kg = 0; kg < 4; ++kg)
 #pragma unroll
             for (int c = 0; c < 2; ++c) acc[c] = __builtin_amdgcn_mfma_f32_4x4x4f16(x, m4_b(wp, c, kg), acc[c], 0, 0, 0);
+        mfma_end<2>();
 #pragma unroll
         for (int i = 0; i <= R::K; ++i) w.b[i] += 0x7F4A7C15u * (i + 1);
     }

@@ -32,7 +32,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict
     LaneWords<R::K> lw;
     load_slice<R::K>(lw, weight_rsrc(trellis + ((size_t)kt * nt_n + nt0) * R::TW), 0, lane_off);
     half2_t wp[16];
-    decode_slice<K2>(lw, sh, wp);
+    decode_slice<K2, true>(lw, sh, wp);
     uint32_t* dst = rows[threadIdx.x >> 6];
     // wp[4 u + 2 c + kh]: column q + 8 c, k = 8 kh + 2 u and + 1; even lanes keep k of columns q, q + 1,
     // odd lanes k + 1 of columns q - 1, q

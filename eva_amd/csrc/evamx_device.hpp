@@ -25,26 +25,100 @@ __device__ __forceinline__ uint32_t funnel(uint32_t hi, uint32_t lo, int s)
     return (uint32_t)((((uint64_t)hi << 32) | lo) >> s);
 }
 
-// MUL1 hash of a 16-bit state sitting in the low (HI=false) or high (HI=true) half of r:
+// MUL1 hashes of the 16-bit states in the low (HI=false) or high (HI=true) halves of two registers:
 // state * 0x83DCD12D mod 2^32, split as state*0xD12D + ((state*0x83DC) mod 2^16) << 16 so that
 // it maps to a 16-bit multiply with a word-1 destination (SDWA) and a 16x16->32 multiply-add,
-// instead of the multi-pass 32-bit multiply.
-// Written in inline asm: the compiler otherwise folds the split back into v_mul_lo_u32, or
-// masks the half with an extra instruction instead of using the 16-bit operand selects.
-template <bool HI>
-__device__ __forceinline__ uint32_t mul1_hash(uint32_t r)
-{
-    uint32_t y, p;
-    if constexpr (HI) {
-        asm("v_mul_lo_u16_sdwa %0, %1, %2 dst_sel:WORD_1 dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:DWORD"
-            : "=v"(y) : "v"(r), "v"(0x83DCu));
-        asm("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(p) : "v"(r), "v"(0xD12Du), "v"(y));
-    } else {
-        asm("v_mul_lo_u16_sdwa %0, %1, %2 dst_sel:WORD_1 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:DWORD"
-            : "=v"(y) : "v"(r), "v"(0x83DCu));
-        asm("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(p) : "v"(r), "v"(0xD12Du), "v"(y));
+// instead of the multi-pass 32-bit multiply. Inline asm, since the compiler otherwise folds the split
+// back into v_mul_lo_u32, or masks the half with an extra instruction instead of using the 16-bit
+// operand selects.
+//
+// The compiler keeps no wait states between inline asm and matrix instructions: an asm that writes a
+// register of its own choosing can write one that a matrix instruction just before it still reads, or has
+// yet to write (tests/test_isa_hazards.py reads the built code for it). So there are two forms:
+//   - FENCED: the caller keeps decode and matrix instructions apart (mfma_begin, mfma_end);
+//   - otherwise, where the two run interleaved, every asm writes a register whose value it takes over: the
+//     multiply-add that of the product it adds, the multiply that of a hash of the previous pair, whose byte
+//     sums are taken by then. The first pair's registers are written by the compiler's own instruction,
+//     a packed multiply whose low half's factor is 0, which gets those waits (and is slower).
+#define EVAMX_MUL "v_mul_lo_u16_sdwa %0, %1, %2 dst_sel:WORD_1 dst_unused:UNUSED_PAD src0_sel:"
+template <bool FENCED>
+struct Mul1 {
+    uint32_t p[2];          // the last two hashes
+
+    // A hash in registers of the compiler's choice (FENCED).
+    template <bool HI>
+    __device__ __forceinline__ static uint32_t hash(uint32_t r)
+    {
+        uint32_t y, h;
+        if constexpr (HI) {
+            asm(EVAMX_MUL "WORD_1 src1_sel:DWORD" : "=v"(y) : "v"(r), "v"(0x83DCu));
+            asm("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(h) : "v"(r), "v"(0xD12Du), "v"(y));
+        } else {
+            asm(EVAMX_MUL "WORD_0 src1_sel:DWORD" : "=v"(y) : "v"(r), "v"(0x83DCu));
+            asm("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(h) : "v"(r), "v"(0xD12Du), "v"(y));
+        }
+        return h;
     }
-    return p;
+    // The product in p[i] becomes the hash.
+    template <bool HI>
+    __device__ __forceinline__ void add(int i, uint32_t r)
+    {
+        if constexpr (HI) asm("v_mad_u32_u16 %0, %1, %2, %0 op_sel:[1,0,0,0]" : "+v"(p[i]) : "v"(r), "v"(0xD12Du));
+        else asm("v_mad_u32_u16 %0, %1, %2, %0" : "+v"(p[i]) : "v"(r), "v"(0xD12Du));
+    }
+    // The first pair. (The factor and the windows are opaque, or the compiler makes one 32-bit product
+    // and shifts the halves out of the words anew.)
+    template <bool HI>
+    __device__ __forceinline__ void first(uint32_t r0, uint32_t r1)
+    {
+        if constexpr (FENCED) {
+            next<HI>(r0, r1);
+        } else {
+            uint32_t c = 0x83DC0000u;
+            asm("" : "+s"(c));
+            asm("" : "+v"(r0), "+v"(r1));
+            const uint32_t r[2] = {r0, r1};
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const u16x2_t s = __builtin_bit_cast(u16x2_t, r[i]);
+                p[i] = __builtin_bit_cast(uint32_t, (HI ? u16x2_t{s.y, s.y} : u16x2_t{s.x, s.x}) * __builtin_bit_cast(u16x2_t, c));
+                add<HI>(i, r[i]);
+            }
+        }
+    }
+    template <bool HI>
+    __device__ __forceinline__ void next(uint32_t r0, uint32_t r1)
+    {
+        const uint32_t r[2] = {r0, r1};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if constexpr (FENCED) {
+                p[i] = hash<HI>(r[i]);
+            } else {
+                if constexpr (HI) asm(EVAMX_MUL "WORD_1 src1_sel:DWORD" : "=v"(p[i]) : "v"(r[i]), "v"(0x83DCu), "0"(p[i]));
+                else asm(EVAMX_MUL "WORD_0 src1_sel:DWORD" : "=v"(p[i]) : "v"(r[i]), "v"(0x83DCu), "0"(p[i]));
+                add<HI>(i, r[i]);
+            }
+        }
+    }
+};
+#undef EVAMX_MUL
+
+// Around the matrix instructions of a fenced decode: no instruction is scheduled across, and the decode
+// that follows starts once none of their registers that it may be given is pending. Those are the ones the
+// last instruction reads its sums from (pending for 1 wait state at 2 passes, 3 at 4), which the one
+// before it may have written (5 and 7, counted from that one); the last one's results are live. The
+// SIMD's other waves issue meanwhile.
+__device__ __forceinline__ void mfma_begin() { __builtin_amdgcn_sched_barrier(0); }
+
+template <int PASSES>
+__device__ __forceinline__ void mfma_end()
+{
+    static_assert(PASSES == 2 || PASSES == 4, "4x4x4 or 16x16x32 matrix instructions");
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (PASSES == 2) asm volatile("s_nop 2");
+    else asm volatile("s_nop 3");
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 // The fp16 pair h = (1024 + bytesum) of two hashes, before the codebook's affine map
@@ -95,31 +169,25 @@ __device__ __forceinline__ uint32_t win_reg(const LaneWords<K>& w)
     return funnel(w.b[L - 1], w.b[L], S);
 }
 
-// Hash of lane-local position j (0..31). When K divides 16, the windows of positions j and
-// j + 16/K are 16 bits apart and share one funnel shift: with P = 16/K, positions in odd
-// P-blocks take the low half of their own register, positions in even P-blocks the high half
-// of the register of j + P.
-template <int K, int J>
-__device__ __forceinline__ uint32_t lane_hash(const LaneWords<K>& w)
+// The (1024 + bytesum) pairs of a lane's 32 positions: wp[j] those of 2 j and 2 j + 1 (same column, k and
+// k + 1; see mul1_hpair), two window registers at a time. When K divides 16, the windows of positions j
+// and j + 16/K are 16 bits apart and share a register, the first in its high half.
+template <int K, bool FENCED, int B = 0>
+__device__ __forceinline__ void lane_pairs(const LaneWords<K>& w, Mul1<FENCED>& m, half2_t (&wp)[16])
 {
-    constexpr int E = win_end<K>(J);
-    if constexpr (16 % K == 0) {
-        constexpr int P = 16 / K;
-        if constexpr ((J / P) % 2 == 0)
-            return mul1_hash<true>(win_reg<K, E + 16>(w));
-        else
-            return mul1_hash<false>(win_reg<K, E>(w));
-    } else {
-        return mul1_hash<false>(win_reg<K, E>(w));
+    constexpr bool SHARED = 16 % K == 0;
+    constexpr int P = SHARED ? 16 / K : 0;
+    constexpr int Q = SHARED ? P : 1;
+    constexpr int J = SHARED ? 2 * B / Q * 2 * P + 2 * B % Q : 2 * B;        // the first window's position
+    const uint32_t r0 = win_reg<K, win_end<K>(J + P)>(w), r1 = win_reg<K, win_end<K>(J + 1 + P)>(w);
+    if constexpr (B == 0) m.template first<SHARED>(r0, r1);
+    else m.template next<SHARED>(r0, r1);
+    wp[J / 2] = mul1_hpair(m.p[0], m.p[1]);
+    if constexpr (SHARED) {
+        m.template next<false>(r0, r1);
+        wp[(J + P) / 2] = mul1_hpair(m.p[0], m.p[1]);
     }
-}
-
-// The (1024 + bytesum) pair of lane-local positions (J, J+1) (J even): same column, k and k+1 (see
-// mul1_hpair).
-template <int K, int J>
-__device__ __forceinline__ half2_t lane_hpair(const LaneWords<K>& w)
-{
-    return mul1_hpair(lane_hash<K, J>(w), lane_hash<K, J + 1>(w));
+    if constexpr (B + 1 < (SHARED ? 8 : 16)) lane_pairs<K, FENCED, B + 1>(w, m, wp);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -137,19 +205,23 @@ constexpr int half_win_end(int j)
 }
 
 template <int B, int J>
-__device__ __forceinline__ uint32_t half_hash(const uint32_t (&N)[B + 1])
+__device__ __forceinline__ uint32_t half_reg(const uint32_t (&N)[B + 1])
 {
     constexpr int E = half_win_end<B>(J);
     constexpr int L = (E - 1) / 32;
     constexpr int S = 32 * (L + 1) - E;
     static_assert(L <= B, "window outside the normalised words");
-    return mul1_hash<false>(funnel(N[L > 0 ? L - 1 : 0], N[L], S));
+    return funnel(N[L > 0 ? L - 1 : 0], N[L], S);
 }
 
-template <int B, int J>
-__device__ __forceinline__ half2_t half_hpair(const uint32_t (&N)[B + 1])
+// lane_pairs at a half rate.
+template <int B, bool FENCED, int J = 0>
+__device__ __forceinline__ void half_pairs(const uint32_t (&N)[B + 1], Mul1<FENCED>& m, half2_t (&wp)[16])
 {
-    return mul1_hpair(half_hash<B, J>(N), half_hash<B, J + 1>(N));
+    if constexpr (J == 0) m.template first<false>(half_reg<B, J>(N), half_reg<B, J + 1>(N));
+    else m.template next<false>(half_reg<B, J>(N), half_reg<B, J + 1>(N));
+    wp[J / 2] = mul1_hpair(m.p[0], m.p[1]);
+    if constexpr (J + 2 < 32) half_pairs<B, FENCED, J + 2>(N, m, wp);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -269,37 +269,21 @@ __device__ __forceinline__ void lane_offsets(int lane, uint32_t& lane_off, uint3
 
 // The (1024 + bytesum) pairs of the lane's 32 positions of one k-slice:
 // wp[4u + 2c + kh] = column q + 8c, k = 8kh + 2u and 8kh + 2u + 1 (low half: even k).
-template <int K2>
+// FENCED: no matrix instruction runs among this decode's (see Mul1).
+template <int K2, bool FENCED>
 __device__ __forceinline__ void decode_slice(LaneWords<Rate<K2>::K>& w, uint32_t sh, half2_t (&wp)[16])
 {
     using R = Rate<K2>;
     constexpr int K = R::K, B = R::B;
     w.b[0] = prev_word<K>(w);
+    Mul1<FENCED> m;
     if constexpr (!R::HALF) {
-#define EVAMX_DEC_UNIT(U)                                \
-        wp[4 * U + 0] = lane_hpair<K, 8 * U + 0>(w);     \
-        wp[4 * U + 1] = lane_hpair<K, 8 * U + 2>(w);     \
-        wp[4 * U + 2] = lane_hpair<K, 8 * U + 4>(w);     \
-        wp[4 * U + 3] = lane_hpair<K, 8 * U + 6>(w);
-        EVAMX_DEC_UNIT(0)
-        EVAMX_DEC_UNIT(1)
-        EVAMX_DEC_UNIT(2)
-        EVAMX_DEC_UNIT(3)
-#undef EVAMX_DEC_UNIT
+        lane_pairs<K, FENCED>(w, m, wp);
     } else {
         uint32_t N[B + 1];
 #pragma unroll
         for (int k = 0; k <= B; ++k) N[k] = __builtin_amdgcn_alignbit(w.b[k], w.b[k + 1], sh);
-#define EVAMX_DEC_UNIT(U)                                \
-        wp[4 * U + 0] = half_hpair<B, 8 * U + 0>(N);     \
-        wp[4 * U + 1] = half_hpair<B, 8 * U + 2>(N);     \
-        wp[4 * U + 2] = half_hpair<B, 8 * U + 4>(N);     \
-        wp[4 * U + 3] = half_hpair<B, 8 * U + 6>(N);
-        EVAMX_DEC_UNIT(0)
-        EVAMX_DEC_UNIT(1)
-        EVAMX_DEC_UNIT(2)
-        EVAMX_DEC_UNIT(3)
-#undef EVAMX_DEC_UNIT
+        half_pairs<B, FENCED>(N, m, wp);
     }
 }
 
@@ -421,8 +405,9 @@ __device__ __forceinline__ void gemv_wave_m4(const uint32_t* __restrict__ trelli
 #pragma unroll
             for (int g = 0; g < NA; ++g) xs.load(g, kt, xa[g]);
             half2_t wp[16];
-            decode_slice<K2>(w, sh, wp);
+            decode_slice<K2, true>(w, sh, wp);
             load_slice<K>(w, rsrc, cbase + (uint32_t)min(kt + PF, last) * slice, lane_off);
+            mfma_begin();
 #pragma unroll
             for (int kg = 0; kg < 4; ++kg)
 #pragma unroll
@@ -432,7 +417,7 @@ __device__ __forceinline__ void gemv_wave_m4(const uint32_t* __restrict__ trelli
                     for (int c = 0; c < 2; ++c)
                         acc[g][c] = __builtin_amdgcn_mfma_f32_4x4x4f16(a, m4_b(wp, c, kg), acc[g][c], 0, 0, 0);
                 }
-            __builtin_amdgcn_sched_barrier(0);
+            mfma_end<2>();
         };
 
         const int n_kt = kt1 - kt0;

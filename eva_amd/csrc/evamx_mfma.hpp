@@ -129,8 +129,9 @@ __device__ __forceinline__ void mfma_accumulate(const uint32_t* __restrict__ tre
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             half2_t wp[16];
-            decode_slice<K2>(ring[j], sh, wp);
+            decode_slice<K2, MB == 1>(ring[j], sh, wp);
             load_slice<K>(ring[j], rsrc, cbase + (uint32_t)(4 * kn) * slice + (uint32_t)(8 * j * TW), lane_off);
+            if constexpr (MB == 1) mfma_begin();
 #pragma unroll
             for (int c = 0; c < 2; ++c)
 #pragma unroll
@@ -141,6 +142,7 @@ __device__ __forceinline__ void mfma_accumulate(const uint32_t* __restrict__ tre
                         acc[mb][2 * j + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a[mb][h]), b,
                                                                                     acc[mb][2 * j + c], 0, 0, 0);
                 }
+            if constexpr (MB == 1) mfma_end<4>();
         }
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
@@ -188,8 +190,9 @@ __device__ __forceinline__ void mfma_pair(const uint32_t* __restrict__ trellis, 
     };
     auto step = [&](int t, LaneWords<K>& w, const u32x4_t (&x)[MB][2], u32x4_t (&y)[MB][2]) {
         load_a(y, t + 2);
+        __builtin_amdgcn_sched_barrier(0);        // the loads first
         half2_t wp[16];
-        decode_slice<K2>(w, sh, wp);
+        decode_slice<K2, false>(w, sh, wp);
         load_w(w, t + 3);
 #pragma unroll
         for (int c = 0; c < 2; ++c)

@@ -33,7 +33,7 @@ template <int K2>
 __device__ __forceinline__ WideOps wide_decode(LaneWords<Rate<K2>::K>& w, uint32_t sh)
 {
     half2_t wp[16];
-    decode_slice<K2>(w, sh, wp);
+    decode_slice<K2, false>(w, sh, wp);
     return WideOps{__builtin_bit_cast(u32x4_t, mfma_b(wp, 0, 0)), __builtin_bit_cast(u32x4_t, mfma_b(wp, 0, 1)),
                    __builtin_bit_cast(u32x4_t, mfma_b(wp, 1, 0)), __builtin_bit_cast(u32x4_t, mfma_b(wp, 1, 1))};
 }

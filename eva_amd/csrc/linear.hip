@@ -198,18 +198,22 @@ __device__ __forceinline__ void lin_gemv_range(const LinParams& p, int cg, int h
         auto step = [&](int t, LaneWords<K> (&w)[NU]) {
             const half8_t a0 = __builtin_bit_cast(half8_t, *(const u32x4_t*)(xrow + 32 * t));
             const half8_t a1 = __builtin_bit_cast(half8_t, *(const u32x4_t*)(xrow + 32 * t + 4));
-            ones = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, bones, ones, 0, 0, 0);
-            ones = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, bones, ones, 0, 0, 0);
 #pragma unroll
             for (int j = 0; j < NU; ++j) {
                 half2_t wp[16];
-                decode_slice<K2>(w[j], sh, wp);
+                decode_slice<K2, true>(w[j], sh, wp);
                 load_w(w[j], t + HV, j);
+                mfma_begin();
+                if (j == 0) {
+                    ones = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, bones, ones, 0, 0, 0);
+                    ones = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, bones, ones, 0, 0, 0);
+                }
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
                     acc[2 * j + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, mfma_b(wp, c, 0), acc[2 * j + c], 0, 0, 0);
                     acc[2 * j + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, mfma_b(wp, c, 1), acc[2 * j + c], 0, 0, 0);
                 }
+                mfma_end<4>();
             }
         };
         if (work)
