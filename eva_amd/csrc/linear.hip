@@ -23,10 +23,12 @@ namespace evamx {
 
 
 constexpr int LIN_GEMV_ROWS = 16;     // lin_gemv_kernel up to this many rows
+constexpr int LIN_GRID_Y = 32768;     // column groups along y of its grid
 
 struct LinParams {
     const half_t* x;
-    int rows, in, out, k2, ks;
+    int rows, in, out, ks;
+    int per;           // 128-chunks of a k-split, or 0 where they differ by one
     const uint32_t* trellis;
     const half_t* suh;
     const half_t* svh;
@@ -55,13 +57,17 @@ __device__ __forceinline__ void lin_load_sv(const LinParams& p, int cg, float (&
 // instructions, and a row's bits do not depend on how many share the call. The
 // four splits' results are added in LDS in order; the quarters meet through memory, and the last
 // workgroup to arrive at the column group's counter adds them in order and runs the output epilogue.
-// Bound by latency: the launch, the first weights, the arrival. (Before: v_dot2 per row and two rows'
-// passes from registers, from three rows on a rotation and an epilogue launch around it. 2048 -> 7168 at 4
-// bpw in a graph, us per call: 1 row 7.6 -> 7.4, 2 rows 9.3 -> 8.6, 8 rows 22.5 -> 9.7, 16 rows 36.6 -> 12.4.)
+// Bound by latency: the launch, the first weights, the arrival. So nothing is computed or loaded on the way
+// to the first weights that the call can do without: no division (the workgroup's place is its grid index,
+// equal splits need none), and where a split is one 128-chunk, as up to 2^26 weights, one chunk's loads
+// and nothing past them. (Against a v_dot2 kernel up to two rows, and three launches from three rows on;
+// 2048 -> 7168 at 4 bpw, 64 copies in a graph, us per call, that / this with divisions and loads past the
+// chunk / this: 1 row 6.84 / 7.16 / 6.27, 2 rows 8.44 / 8.05 / 7.25, 8 rows 21.0 / 8.9 / 7.7, 16 rows 35.7 / 11.3
+// / 9.3; 5120 -> 5120 at 3.5 bpw, 1 row 10.2 / 9.5 / 9.0; 1024 -> 18432 at 4 bpw, 1 row 8.5 / 9.4 / 7.9.)
 
 // 128-chunks of rotated rows in LDS at a time, and words of a row there (padded, so that the 16 rows an
-// operand reads lie in different banks). One row: each wave rotates it for itself; more: the two waves of
-// a split rotate half the rows each.
+// operand reads lie in different banks). One row: each wave rotates it for itself; more: the waves of a
+// split share the rows (LinRot).
 template <int TM>
 struct LinStage {
     static constexpr int CW = TM == 1 ? 4 : 2;
@@ -69,33 +75,33 @@ struct LinStage {
     static constexpr int WORDS = TM == 1 ? ROW : TM * ROW;
 };
 
-// fp16(H128(fp16(x * suh))) of the call's rows over the 128-chunks [w0, w1) into LDS. issue() loads ahead
-// of the weight prefetch, finish() rotates behind it. One row: a chunk on the whole wave; more: 16 lanes
-// a chunk, four (row, chunk) pairs at a time. The same bits either way.
-template <int TM>
+// fp16(H128(fp16(x * suh))) of the call's rows over the 128-chunks [w0, w1) into LDS, NC of them at most.
+// issue() loads ahead of the weight prefetch, finish() rotates behind it. One row: a chunk on the whole
+// wave; more: 16 lanes a chunk, four (row, chunk) pairs at a time, the split's HV waves taking turns. The
+// same bits either way.
+template <int TM, int NC, int HV>
 struct LinRot;
 
-template <>
-struct LinRot<1> {
-    uint32_t xv[4], sv[4];
+template <int NC, int HV>
+struct LinRot<1, NC, HV> {
+    uint32_t xv[NC], sv[NC];
     __device__ __forceinline__ void issue(const LinParams& p, int w0, int w1, int)
     {
         const int lane = threadIdx.x & 63;
         const __amdgpu_buffer_rsrc_t xrs = weight_rsrc((const uint32_t*)p.x), srs = weight_rsrc((const uint32_t*)p.suh);
         // chunks past the window reload its last one (in bounds, unused): no branches
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < NC; ++j) {
             const uint32_t off = 256u * (uint32_t)min(w0 + j, w1 - 1);
             sv[j] = __builtin_amdgcn_raw_buffer_load_b32(srs, 4 * lane, off, 0);
             xv[j] = __builtin_amdgcn_raw_buffer_load_b32(xrs, 4 * lane, off, 0);
         }
     }
-    template <int HV>
     __device__ __forceinline__ void finish(const LinParams&, int w0, int w1, int, uint32_t* dst)
     {
         const int lane = threadIdx.x & 63;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < NC; ++j) {
             if (w0 + j < w1) {
                 const half2_t xx = __builtin_bit_cast(half2_t, xv[j]), su = __builtin_bit_cast(half2_t, sv[j]);
                 float v0 = h2f(f2h(h2f(xx.x) * h2f(su.x)));      // fp16 product
@@ -108,31 +114,36 @@ struct LinRot<1> {
     }
 };
 
-template <>
-struct LinRot<16> {
-    u32x4w xv[4], sv[4];
-    __device__ __forceinline__ void load(const LinParams& p, int w0, int w1, int b)
+template <int NC, int HV>
+struct LinRot<16, NC, HV> {
+    static_assert(NC <= 2, "a pair's row and chunk by a shift");
+    static constexpr int NG = LIN_GEMV_ROWS * NC / (4 * HV);     // groups of four pairs a wave at most
+    static constexpr int NL = NG < 4 ? NG : 4;                   // of them loaded at a time
+    u32x4w xv[NL], sv[NL];
+    // pair it: row it >> (nw - 1), chunk w0 + (it & (nw - 1)), for a window of nw (1 or 2) chunks
+    __device__ __forceinline__ void load(const LinParams& p, int w0, int w1, int half, int g0)
     {
-        const int lane = threadIdx.x & 63, nw = w1 - w0, n = p.rows * nw;
+        const int lane = threadIdx.x & 63, sh = NC == 1 ? 0 : w1 - w0 - 1, n = p.rows << sh;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int it = min(b + 4 * i + (lane >> 4), n - 1), m = it / nw, c = w0 + it % nw;
-            const size_t k = 128 * c + 8 * oct_piece(lane);
-            xv[i] = *(const __attribute__((address_space(1))) u32x4w*)(p.x + (size_t)m * p.in + k);
+        for (int i = 0; i < NL; ++i) {
+            const int b = 4 * (HV * (g0 + i) + half);
+            if (b >= n) break;
+            const int it = min(b + (lane >> 4), n - 1);
+            const size_t k = 128 * (w0 + (it & sh)) + 8 * oct_piece(lane);
+            xv[i] = *(const __attribute__((address_space(1))) u32x4w*)(p.x + (size_t)(it >> sh) * p.in + k);
             sv[i] = *(const __attribute__((address_space(1))) u32x4w*)(p.suh + k);
         }
     }
-    __device__ __forceinline__ void issue(const LinParams& p, int w0, int w1, int half) { load(p, w0, w1, 16 * half); }
-    template <int HV>
+    __device__ __forceinline__ void issue(const LinParams& p, int w0, int w1, int half) { load(p, w0, w1, half, 0); }
     __device__ __forceinline__ void finish(const LinParams& p, int w0, int w1, int half, uint32_t* dst)
     {
-        const int lane = threadIdx.x & 63, nw = w1 - w0, n = p.rows * nw;
-        for (int b = 16 * half; b < n; b += 16 * HV) {
-            if (b >= 16 * HV) load(p, w0, w1, b);
+        const int lane = threadIdx.x & 63, sh = NC == 1 ? 0 : w1 - w0 - 1, n = p.rows << sh;
+        for (int g0 = 0; g0 < NG && 4 * (HV * g0 + half) < n; g0 += NL) {
+            if (g0 > 0) load(p, w0, w1, half, g0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int it = b + 4 * i + (lane >> 4);
-                if (b + 4 * i >= n) break;
+            for (int i = 0; i < NL; ++i) {
+                const int b = 4 * (HV * (g0 + i) + half), it = b + (lane >> 4);
+                if (b >= n) break;
                 const uint32_t xu[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w}, su[4] = {sv[i].x, sv[i].y, sv[i].z, sv[i].w};
                 float x[8], h[8];
                 oct_halves(xu, x);
@@ -143,23 +154,24 @@ struct LinRot<16> {
                 u32x4 r;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) r[e] = __builtin_bit_cast(uint32_t, half2_t{f2h(x[2 * e]), f2h(x[2 * e + 1])});
-                if (it < n) *(u32x4*)(dst + (it / nw) * LinStage<16>::ROW + 64 * (it % nw) + 4 * oct_piece(lane)) = r;
+                if (it < n) *(u32x4*)(dst + (it >> sh) * LinStage<16>::ROW + 64 * (it & sh) + 4 * oct_piece(lane)) = r;
             }
         }
     }
 };
 
-// The wave's share of the columns (128 / HV from 128 / HV * half on) over its split's k-range [c0, c1) (128-chunks, none for
-// a wave past the splits): acc[nb][r] = sum_k x_k h_k, ones[r] = sum_k x_k for row 4 g + r and column
-// 128 / HV * half + mfma_col(lane, nb). Every wave of the workgroup runs `windows` windows of CW chunks.
-template <int K2, int TM, int HV>
+// The wave's share of the columns (128 / HV from 128 / HV * half on) over its split's k-range [c0, c1)
+// (128-chunks, none for a wave past the splits): acc[nb][r] = sum_k x_k h_k, ones[r] = sum_k x_k for row
+// 4 g + r and column 128 / HV * half + mfma_col(lane, nb), in windows of NC chunks (TM > 1: every wave of
+// the workgroup runs as many), HV steps of weights in flight. NC 1: every split is one chunk, and
+// nothing past it is loaded.
+template <int K2, int TM, int HV, int NC>
 __device__ __forceinline__ void lin_gemv_range(const LinParams& p, int cg, int half, int c0, int c1, int windows, uint32_t* lds,
                                                f32x4_t (&acc)[8 / HV], f32x4_t& ones)
 {
     using R = Rate<K2>;
     constexpr int K = R::K;
     constexpr int TW = R::TW;
-    constexpr int CW = LinStage<TM>::CW;
     constexpr int NU = 4 / HV;                            // units (pairs of tiles) a step
     const int lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4, nt_n = p.out / 16;
     const uint32_t slice = __builtin_amdgcn_readfirstlane(4u * (uint32_t)(nt_n * TW));
@@ -176,7 +188,7 @@ __device__ __forceinline__ void lin_gemv_range(const LinParams& p, int cg, int h
     for (int nb = 0; nb < 2 * NU; ++nb) acc[nb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     ones = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     for (int i = 0; i < windows; ++i) {
-        const int w0 = c0 + i * CW, w1 = min(c1, w0 + CW), steps = 2 * (w1 - w0);
+        const int w0 = c0 + i * NC, w1 = min(c1, w0 + NC), steps = NC == 1 ? 2 : 2 * (w1 - w0);
         const uint32_t wbase = cbase + (uint32_t)(8 * w0) * slice;
         const bool work = w0 < w1;                        // wave-uniform
         LaneWords<K> ring[HV][NU];                        // HV steps
@@ -184,14 +196,14 @@ __device__ __forceinline__ void lin_gemv_range(const LinParams& p, int cg, int h
             load_slice<K>(w, rsrc, wbase + (uint32_t)(4 * min(t, steps - 1)) * slice + (uint32_t)(8 * j * TW), lane_off);
         };
         if (work) {
-            LinRot<TM> rot;
+            LinRot<TM, NC, HV> rot;
             rot.issue(p, w0, w1, half);
 #pragma unroll
             for (int t = 0; t < HV; ++t)
 #pragma unroll
                 for (int j = 0; j < NU; ++j) load_w(ring[t][j], t, j);
             __builtin_amdgcn_sched_barrier(0);
-            rot.template finish<HV>(p, w0, w1, half, lds);
+            rot.finish(p, w0, w1, half, lds);
         }
         if constexpr (TM == 1) wave_lds_fence();
         else __syncthreads();
@@ -202,7 +214,7 @@ __device__ __forceinline__ void lin_gemv_range(const LinParams& p, int cg, int h
             for (int j = 0; j < NU; ++j) {
                 half2_t wp[16];
                 decode_slice<K2, true>(w[j], sh, wp);
-                load_w(w[j], t + HV, j);
+                if (NC > 1 || t + HV < steps) load_w(w[j], t + HV, j);
                 mfma_begin();
                 if (j == 0) {
                     ones = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, bones, ones, 0, 0, 0);
@@ -294,16 +306,23 @@ __global__ __launch_bounds__(256 * HV) __attribute__((amdgpu_waves_per_eu(TM == 
     __shared__ float res1[TM == 1 ? 4 : 1][128];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63, g = lane >> 4;
     const int split = wave / HV, half = wave % HV;
-    const int nq = (p.ks + 3) >> 2;
-    const int cg = blockIdx.x / nq, q = blockIdx.x % nq;
+    // q fastest: the workgroups of a column group side by side
+    const int nq = (p.ks + 3) >> 2, q = blockIdx.x, cg = blockIdx.y + LIN_GRID_Y * blockIdx.z;
+    if (cg >= p.out / 128) return;
     const int ks = 4 * q + split, nv = min(4, p.ks - 4 * q);     // the workgroup's splits
     float sv[2];
     lin_load_sv(p, cg, sv);
-    const int nch = p.in / 128;
-    const int c0 = split < nv ? nch * ks / p.ks : 0, c1 = split < nv ? nch * (ks + 1) / p.ks : 0;
-    const int windows = ((nch + p.ks - 1) / p.ks + LinStage<TM>::CW - 1) / LinStage<TM>::CW;
     f32x4_t acc[8 / HV], ones;
-    lin_gemv_range<K2, TM, HV>(p, cg, half, c0, c1, windows, lds[TM == 1 ? wave : split], acc, ones);
+    uint32_t* const stage = lds[TM == 1 ? wave : split];
+    if (p.per == 1) {
+        lin_gemv_range<K2, TM, HV, 1>(p, cg, half, ks, split < nv ? ks + 1 : ks, 1, stage, acc, ones);
+    } else {
+        constexpr int CW = LinStage<TM>::CW;
+        const int nch = p.in / 128;
+        const int c0 = split < nv ? nch * ks / p.ks : 0, c1 = split < nv ? nch * (ks + 1) / p.ks : 0;
+        const int most = TM == 1 ? c1 - c0 : (nch + p.ks - 1) / p.ks;
+        lin_gemv_range<K2, TM, HV, CW>(p, cg, half, c0, c1, (most + CW - 1) / CW, stage, acc, ones);
+    }
     auto res = [&](int w) { return TM == 1 ? res1[w] : (float*)lds[w]; };        // split w's results [row][128]
     if (split < nv) {
         float* d = res(split) + 128 / HV * half;
@@ -318,8 +337,11 @@ __global__ __launch_bounds__(256 * HV) __attribute__((amdgpu_waves_per_eu(TM == 
     }
     __syncthreads();
     auto sum = [&](int i) {                                      // the splits' result i, in split order
-        float t = res(0)[i];
-        for (int w = 1; w < nv; ++w) t += res(w)[i];
+        const float t0 = res(0)[i], t1 = res(min(1, nv - 1))[i], t2 = res(min(2, nv - 1))[i], t3 = res(nv - 1)[i];
+        float t = t0;
+        if (nv > 1) t += t1;
+        if (nv > 2) t += t2;
+        if (nv > 3) t += t3;
         return t;
     };
     if (nq == 1) {
@@ -353,14 +375,14 @@ __global__ __launch_bounds__(256 * HV) __attribute__((amdgpu_waves_per_eu(TM == 
 }
 
 // Decode path launch of one rate: workgroups per (column group, four splits), of eight waves while one
-// workgroup a CU leaves the SIMDs a wave each otherwise, of four beyond (5120 x 5120 at 5 bpw, 400
-// workgroups: one row 11.3 against 12.6 us, 13 rows 16.0 against 20.0; 7168 -> 2048 at 2.5 bpw, 224: one row
-// 7.7 against 7.3, 8 rows 11.0 against 10.1).
+// workgroup a CU leaves the SIMDs a wave each otherwise, of four beyond (four waves against eight: 5120 ->
+// 5120 at 5 bpw, 400 workgroups, one row 9.8 against 10.0 us, 13 rows 14.9 against 18.4; 7168 -> 2048 at 2.5
+// bpw, 224, one row 6.9 against 6.6, 8 rows 10.8 against 8.8).
 template <int K2>
 void launch_gemv_rate(const LinParams& p, hipStream_t stream)
 {
-    const int blocks = p.out / 128 * ((p.ks + 3) / 4);
-    const dim3 grid((unsigned)blocks);
+    const int ncg = p.out / 128, nq = (p.ks + 3) / 4, blocks = ncg * nq;
+    const dim3 grid((unsigned)nq, (unsigned)std::min(ncg, LIN_GRID_Y), (unsigned)((ncg + LIN_GRID_Y - 1) / LIN_GRID_Y));
     if (blocks <= 256) {
         if (p.rows == 1) hipLaunchKernelGGL((lin_gemv_kernel<K2, 1, 2>), grid, dim3(512), 0, stream, p);
         else hipLaunchKernelGGL((lin_gemv_kernel<K2, 16, 2>), grid, dim3(512), 0, stream, p);
@@ -743,8 +765,9 @@ int launch_linear(const void* x, int rows, int in, int out, const void* trellis,
     linear_workspace(rows, in, out, &off_part, &off_sum);
     const int kind_ws = rows > LIN_GEMV_ROWS ? linear_kind(rows, in, out, k2) : -1;
     p.x = (const half_t*)x;
-    p.rows = rows; p.in = in; p.out = out; p.k2 = k2;
+    p.rows = rows; p.in = in; p.out = out;
     p.ks = linear_ksplit(rows, in, out);
+    p.per = in / 128 % p.ks == 0 ? in / 128 / p.ks : 0;
     p.trellis = (const uint32_t*)trellis;
     p.suh = (const half_t*)suh;
     p.svh = (const half_t*)svh;

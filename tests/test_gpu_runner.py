@@ -153,8 +153,8 @@ def test_linear_row_kernels(dev, shape, K, counts):
 
 @pytest.mark.parametrize("shape,K", [((128, 128), 4), ((512, 256), 2), ((640, 1024), 3.5), ((5120, 5120), 5), ((1280, 40960), 1.5)])
 def test_linear_decode_rows_bit_identical(dev, shape, K):
-    """1 to 16 rows: one k-split quarter and many, workgroups of four and of eight waves, one and several
-    128-chunks a split. Every row has the bits of its one-row call; those are held to the oracle."""
+    """1 to 16 rows, one 128-chunk a split: one k-split quarter and many, workgroups of four and of eight
+    waves. Every row has the bits of its one-row call; those are held to the oracle."""
     n_in, n_out = shape
     rng = np.random.default_rng(n_in + n_out)
     tr, suh, svh = synth.projection(rng, n_in, n_out, K, n_in ** -0.5)
@@ -165,9 +165,40 @@ def test_linear_decode_rows_bit_identical(dev, shape, K):
     one = torch.cat([lin.forward(xd[r:r + 1]) for r in range(16)])
     for rows in (2, 3, 4, 5, 7, 8, 9, 13, 16):
         assert torch.equal(lin.forward(xd[:rows]).view(torch.int16), one[:rows].view(torch.int16)), rows
-    if n_out <= 5120:
-        ref = coop.exl3_linear(x[:2], tr, suh, svh, K)
-        assert rel_err_rows(one[:2].cpu().numpy().astype(np.float32), ref.astype(np.float32)) < TOL
+    _check_columns(one[:2], x[:2], tr, suh, svh, K, [range(0, min(n_out, 5120) // 128)])
+
+
+def _check_columns(y, x, tr, suh, svh, K, spans):
+    """Some 128-column groups of y = linear(x) against the oracle: a group depends on its own tiles only."""
+    for groups in spans:
+        a, b = 128 * groups[0], 128 * (groups[-1] + 1)
+        ref = coop.exl3_linear(x, np.ascontiguousarray(tr[:, a // 16:b // 16]), suh, svh[a:b], K)
+        assert rel_err_rows(y[:, a:b].cpu().numpy().astype(np.float32), ref.astype(np.float32)) < TOL, a
+
+
+@pytest.mark.parametrize("shape,K", [
+    ((7168, 18432), 1.5),        # 56 chunks over 29 splits: one or two each
+    ((18432, 7168), 3),          # 144 over 74
+    ((1152, 524288), 1.5),       # nine chunks in one split: three windows of four, five of two
+    ((512, 65536), 5),           # one chunk a split, one quarter
+    ((128, 4194432), 1.5),       # more column groups than a grid's second dimension takes
+])
+def test_linear_decode_rows_wide(dev, shape, K):
+    """1 to 16 rows where a split has several 128-chunks, evenly and unevenly, in one LDS window and in
+    several, and at the largest column counts. Every row has the bits of its one-row call; some column
+    groups of those are held to the oracle."""
+    n_in, n_out = shape
+    rng = np.random.default_rng(n_in + n_out)
+    tr, suh, svh = synth.projection(rng, n_in, n_out, K, n_in ** -0.5)
+    from eva_amd.linear import build_linear
+    lin = build_linear(to_dev(suh, dev), to_dev(svh, dev), to_dev(tr, dev), device=dev)
+    x = rng.standard_normal((16, n_in)).astype(np.float16)
+    xd = to_dev(x, dev)
+    one = torch.cat([lin.forward(xd[r:r + 1]) for r in range(16)])
+    for rows in (2, 5, 9, 16):
+        assert torch.equal(lin.forward(xd[:rows]).view(torch.int16), one[:rows].view(torch.int16)), rows
+    n = n_out // 128
+    _check_columns(one[:2], x[:2], tr, suh, svh, K, [range(g, g + 1) for g in sorted({0, 1, n // 2, n - 2, n - 1})])
 
 
 @pytest.mark.parametrize("rows", [1, 13])
