@@ -646,34 +646,35 @@ __global__ __launch_bounds__(64 * LW_WAVES) __attribute__((amdgpu_waves_per_eu(2
     }
 }
 
-// Whether a call's 64-row workgroups take one k-range each: while they are few (their partials cost more
-// the more tiles there are, the others' latency the longer k). us per call split / all ranges at 4 bpw in a
-// graph: 2048 -> 7168, 64 rows 20 / 32, 128 rows 33 / 33; 7168 -> 2048, 256 rows 33 / 74, 768 rows 75 / 78;
-// 18432 -> 7168, 320 rows 217 / 285, 512 rows 327 / 292. By size only: the workspace depends on it.
+// Whether a call's 64-row workgroups take one k-range each: while their 16-row blocks are few (the ranges'
+// partials and products grow with them, the others' latency with k). us per call split / all ranges at 4
+// bpw in a graph: 2048 -> 7168, 64 rows 23 / 30, 128 rows 32 / 31; 7168 -> 2048, 512 rows 52 / 69, 768 rows 78 /
+// 75; 7168 -> 18432, 65 rows 76 / 86, 129 rows 125 / 117; 18432 -> 7168, 224 rows 156 / 156, 256 rows 175 / 162.
+// By size only: the workspace depends on it.
 static bool linear_splits(int rows, int in, int out)
 {
     // up to 32 rows and 1024 inputs an eager call is launches: one less (17.0 against 19.0 us)
     if (rows <= 32 && in <= 1024) return false;
-    return (long)((rows + LM_ROWS - 1) / LM_ROWS) * (out / 128) < 80 + in / 76;
+    return (long)((rows + 15) / 16) * (out / 128) < 240 + in / 14;
 }
 
 // Kernel of a call of more than LIN_GEMV_ROWS rows. Wide tiles pay off once they fill the device, the
 // earlier the longer k is (a wide workgroup's fixed cost is its epilogue), if their rows are there: a wide
 // workgroup of a few rows takes as long as a full one, so the 64-row workgroups, which count the rows that
 // there are, have to fill the device (256 workgroups) about twice for each time the wide ones do; somewhat
-// less from 7168 inputs on, where two of the former on a CU take as long as one wide one, and at 5 bpw, whose
-// decode (five words a lane, no shared funnel shifts) costs a quarter more. us per call split / all ranges /
-// wide in a graph: 7168 -> 18432 at 4 bpw, 17 rows 44 / 59 / 109, 128 rows 102 / 116 / 112, 257 rows - / 171 /
-// 218, 512 rows - / 297 / 234, at 5 bpw 128 rows 124 / 143 / 114; 4096 -> 14336 at 3.5 bpw, 64 rows 39 / 52 /
-// 78, 320 rows - / 108 / 84; 7168 -> 7168 at 2.5 to 4 bpw, 257 rows 92 / 82 / 112, 384 rows 119 / 114 / 114;
-// 2048 -> 12288, 640 rows - / 78 / 99; 7168 -> 2048, 1024 rows 98 / 80 / 116, 2048 rows - / 133 / 127; 384 ->
-// 40960 (2.5 bpw), 257 rows - / 44 / 70; 1024 -> 1024, 2048 rows 51 / 34 / 44.
+// less from 7168 inputs on, where two of the former on a CU take as long as one wide one. us per call split /
+// all ranges / wide in a graph: 7168 -> 18432 at 4 bpw, 17 rows 41 / 53 / 111, 128 rows 108 / 114 / 117, 257
+// rows - / 173 / 229, 512 rows - / 298 / 246, at 5 bpw 17 rows 51 / 60 / 118, 128 rows 127 / 145 / 122, 512 rows
+// - / 374 / 259; 4096 -> 14336 at 3.5 bpw, 64 rows 40 / 46 / 76, 320 rows - / 104 / 86; 7168 -> 7168 at 4 bpw, 257
+// rows 91 / 82 / 117, 384 rows 121 / 114 / 118, 640 rows - / 168 / 121; 2048 -> 12288, 640 rows - / 78 / 102;
+// 7168 -> 2048, 1024 rows 103 / 79 / 121, 2048 rows - / 145 / 139; 384 -> 40960 at 2.5 bpw, 257 rows - / 44 / 70;
+// 1024 -> 1024, 2048 rows 52 / 33 / 44.
 enum { LIN_SPLIT, LIN_FULL, LIN_WIDE };
-static int linear_kind(int rows, int in, int out, int k2)
+static int linear_kind(int rows, int in, int out)
 {
     const long ncg = out / 128, wide = (rows + LW_ROWS - 1) / LW_ROWS * ncg, mid = (rows + LM_ROWS - 1) / LM_ROWS * ncg;
-    const float k = (float)in / 1024, rounds = (float)((wide + 255) / 256);
-    const float fill = (rounds * (2.0f + 0.5f / k) - (k >= 7.0f ? 0.75f : 0.0f)) * (k2 == 10 ? 0.75f : 1.0f);
+    const float rounds = (float)((wide + 255) / 256);
+    const float fill = rounds * (2.0f + 300.0f / in) - (in >= 7168 ? 0.75f : 0.0f);
     if (wide >= 80 + 114688 / in && (float)mid >= 256.0f * fill) return LIN_WIDE;
     return linear_splits(rows, in, out) ? LIN_SPLIT : LIN_FULL;
 }
@@ -746,7 +747,7 @@ size_t linear_workspace_upto(int rows, int in, int out)
     };
     most(LIN_GEMV_ROWS);
     // the last row count that may be split (linear_splits' line)
-    const long ncg = out / 128, full = 80 + in / 76, last = ((full + ncg - 1) / ncg - 1) * LM_ROWS;
+    const long ncg = out / 128, full = 240 + in / 14, last = ((full + ncg - 1) / ncg - 1) * 16;
     if (last > LIN_GEMV_ROWS) most((int)std::min(last, 65536L));
     return n;
 }
@@ -763,7 +764,7 @@ int launch_linear(const void* x, int rows, int in, int out, const void* trellis,
     LinParams p;
     size_t off_part, off_sum;
     linear_workspace(rows, in, out, &off_part, &off_sum);
-    const int kind_ws = rows > LIN_GEMV_ROWS ? linear_kind(rows, in, out, k2) : -1;
+    const int kind_ws = rows > LIN_GEMV_ROWS ? linear_kind(rows, in, out) : -1;
     p.x = (const half_t*)x;
     p.rows = rows; p.in = in; p.out = out;
     p.ks = linear_ksplit(rows, in, out);
