@@ -288,9 +288,8 @@ __device__ __forceinline__ void decode_slice(LaneWords<Rate<K2>::K>& w, uint32_t
 }
 
 // ---------------------------------------------------------------------------------------------
-// Activation rows of a GEMV chunk: row m holds the k-vector of slot slot_of[m], read through
-// wave-uniform addresses (scalar loads), together with its per-128-chunk sums (fp32) that the
-// affine codebook map needs.
+// Activation rows of the MFMA tiles: the k-vector of each slot, which a tile's lanes read as their A
+// operands, together with its per-128-chunk sums (fp32) that the affine codebook map needs.
 
 struct GlobalRows {
     const half_t* A;

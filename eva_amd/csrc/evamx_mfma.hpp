@@ -74,7 +74,10 @@ __device__ __forceinline__ void had128_acc(float (&v)[8], int lane)
 // (fp16 [slot][K] with 128-chunk sums) times the (1024 + bytesum) values of tiles 8*cg .. 8*cg+7
 // of a projection over the k-slices [kt0, kt1) (whole 128-chunks): acc[mb][nb][r] = sum_k x_k h_k
 // for row 16 mb + 4 g + r and column mfma_col(lane, nb) (lane = m16 + 16 g).
-template <int K2, int MB, bool PRIO>
+// One row block decodes apart from the products, more interleaved with them (Mul1): fenced, a unit's four
+// operands and four blocks' rows are all live at once and spill (3001 tokens 5404 against 5193 us), interleaved
+// one block is slower (100 tokens at 3 bpw 1454 against 1410).
+template <int K2, int MB>
 __device__ __forceinline__ void mfma_accumulate(const uint32_t* __restrict__ trellis, int nt_n, int cg, int kt0, int kt1,
                                                 const GlobalRows& src, const int* __restrict__ slot_of, int rows,
                                                 f32x4_t (&acc)[MB][8])
@@ -118,7 +121,7 @@ __device__ __forceinline__ void mfma_accumulate(const uint32_t* __restrict__ tre
         for (int h = 0; h < 2; ++h) a[mb][h] = arow[mb][h];
 
     for (int kk = 0; kk < steps; ++kk) {
-        if constexpr (PRIO) progress_priority(kk, steps);
+        progress_priority(kk, steps);
         // the next step's A operands and weights, clamped to the last step (in bounds, unused)
         const int kn = kk + 1 < steps ? kk + 1 : kk;
         u32x4_t an[MB][2];
@@ -149,7 +152,7 @@ __device__ __forceinline__ void mfma_accumulate(const uint32_t* __restrict__ tre
 #pragma unroll
             for (int h = 0; h < 2; ++h) a[mb][h] = an[mb][h];
     }
-    if constexpr (PRIO) progress_priority(1, 1);
+    progress_priority(1, 1);
 }
 
 // Activations laid out as A operands: a block of 16 rows is, for each k64 step t and k half h, the 64
@@ -252,13 +255,13 @@ __device__ __forceinline__ void mfma_row_sums(const GlobalRows& src, const int* 
 
 // One work item with its partials stored: part[slot * part_stride + 128 * cg + column] =
 // 0x1eee * acc + 0xc931 * (row's activation sum), for rows < rows.
-template <int K2, int MB, bool PRIO>
+template <int K2, int MB>
 __device__ __forceinline__ void mfma_item(const uint32_t* __restrict__ trellis, int nt_n, int cg, int kt0, int kt1,
                                           const GlobalRows& src, const int* __restrict__ slot_of, int rows,
                                           float* __restrict__ part, size_t part_stride)
 {
     f32x4_t acc[MB][8];
-    mfma_accumulate<K2, MB, PRIO>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, acc);
+    mfma_accumulate<K2, MB>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, acc);
     kt0 = __builtin_amdgcn_readfirstlane(kt0);
     const int nk = __builtin_amdgcn_readfirstlane(kt1) - kt0;
     float xs[MB][4];

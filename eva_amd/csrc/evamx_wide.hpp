@@ -1,7 +1,7 @@
-// Wide tiles: a workgroup of NW (4 or 8) waves multiplies up to 16 MB NW rows by 128 columns with every
+// Wide tiles: a workgroup of WIDE_WAVES waves multiplies up to 16 MB rows a wave by 128 columns with every
 // weight decoded once for all of them.
 //
-// Per stage of 16 NW k (NW k-slices) each wave decodes one unit (a pair of the column group's tiles over
+// Per stage of 128 k (8 k-slices) each wave decodes one unit (a pair of the column group's tiles over
 // 4 k-slices) into its four B operands (evamx_mfma.hpp: the decode's own register layout) and stores
 // them to LDS as they are, 16 bytes a lane; all waves then multiply all the operands by their own rows'
 // A operands, read straight from global memory. Operands alternate between two LDS buffers, so a stage needs one
@@ -11,9 +11,10 @@
 
 namespace evamx {
 
-template <int NW>
+constexpr int WIDE_WAVES = 8;
+
 struct WideLds {
-    u32x4_t b[2][4 * NW][64];       // [buffer][4 unit + 2 c + h][lane]; unit 4 i + j: pair j at k64 step i
+    u32x4_t b[2][4 * WIDE_WAVES][64];       // [buffer][4 unit + 2 c + h][lane]; unit 4 i + j: pair j at k64 step i
 };
 
 // LDS stores before the barrier are visible after it; loads from global memory stay in flight.
@@ -38,8 +39,7 @@ __device__ __forceinline__ WideOps wide_decode(LaneWords<Rate<K2>::K>& w, uint32
                    __builtin_bit_cast(u32x4_t, mfma_b(wp, 1, 0)), __builtin_bit_cast(u32x4_t, mfma_b(wp, 1, 1))};
 }
 
-template <int NW>
-__device__ __forceinline__ void wide_put(WideLds<NW>& lds, int buf, int unit, int lane, const WideOps& o)
+__device__ __forceinline__ void wide_put(WideLds& lds, int buf, int unit, int lane, const WideOps& o)
 {
     lds.b[buf][4 * unit][lane] = o.o0;
     lds.b[buf][4 * unit + 1][lane] = o.o1;
@@ -50,19 +50,17 @@ __device__ __forceinline__ void wide_put(WideLds<NW>& lds, int buf, int unit, in
 // acc[mb][nb][r] += sum_k x_k h_k over `chunks` 128-chunks of k from k-slice kt0 on, for row 4 g + r of
 // the 16-row block mb (its A operands at arow[mb], a_operand_offset) and column mfma_col(lane, nb).
 // end(c) runs after chunk c.
-template <int K2, int MB, int NW, typename End>
+template <int K2, int MB, typename End>
 __device__ __forceinline__ void wide_accumulate(const uint32_t* __restrict__ trellis, int nt_n, int cg, int kt0, int chunks,
                                                 const __attribute__((address_space(1))) u32x4_t* const (&arow)[MB],
-                                                WideLds<NW>& lds, f32x4_t (&acc)[MB][8], End&& end)
+                                                WideLds& lds, f32x4_t (&acc)[MB][8], End&& end)
 {
     using R = Rate<K2>;
     constexpr int K = R::K;
     constexpr int TW = R::TW;
-    constexpr int SUB = NW / 4;                   // k64 steps per stage
-    static_assert(NW == 4 || NW == 8, "4 or 8 waves");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int g = lane >> 4;
-    const int stages = chunks * (2 / SUB), last = stages - 1, last_step = 2 * chunks - 1;
+    const int last = chunks - 1, last_step = 2 * chunks - 1;       // a stage is a chunk, of two k64 steps
     const uint32_t slice = __builtin_amdgcn_readfirstlane(4u * (uint32_t)(nt_n * TW));
     const uint32_t cbase = __builtin_amdgcn_readfirstlane(4u * (uint32_t)((cg * 8 + 2 * (wave & 3)) * TW) +
                                                           (uint32_t)(kt0 + 4 * (wave >> 2)) * slice);
@@ -80,7 +78,7 @@ __device__ __forceinline__ void wide_accumulate(const uint32_t* __restrict__ tre
             for (int h = 0; h < 2; ++h) d[mb][h] = arow[mb][128 * min(t, last_step) + 64 * h];
     };
     auto load_w = [&](LaneWords<K>& w, int s) {
-        load_slice<K>(w, rsrc, cbase + (uint32_t)(NW * min(s, last)) * slice, lane_off);
+        load_slice<K>(w, rsrc, cbase + (uint32_t)(8 * min(s, last)) * slice, lane_off);
     };
     load_w(ring[0], 0);
     load_w(ring[1], 1);
@@ -105,31 +103,21 @@ __device__ __forceinline__ void wide_accumulate(const uint32_t* __restrict__ tre
     // stage s from buffer buf, while the next stage's unit w is decoded into the other buffer (past the
     // end: a repeat, unused); activations are loaded one k64 step ahead, weights two stages
     auto stage = [&](int s, int buf, LaneWords<K>& w) {
-        if constexpr (SUB == 2) {
-            load_a(a[1], 2 * s + 1);
-            const WideOps o = wide_decode<K2>(w, sh);
-            load_w(w, s + 3);
-            products(buf, 0, a[0]);
-            load_a(a[0], 2 * s + 2);
-            products(buf, 1, a[1]);
-            wide_put(lds, buf ^ 1, wave, lane, o);
-        } else {
-            load_a(a[buf ^ 1], s + 1);
-            const WideOps o = wide_decode<K2>(w, sh);
-            load_w(w, s + 3);
-            products(buf, 0, a[buf]);
-            wide_put(lds, buf ^ 1, wave, lane, o);
-        }
+        load_a(a[1], 2 * s + 1);
+        const WideOps o = wide_decode<K2>(w, sh);
+        load_w(w, s + 3);
+        products(buf, 0, a[0]);
+        load_a(a[0], 2 * s + 2);
+        products(buf, 1, a[1]);
+        wide_put(lds, buf ^ 1, wave, lane, o);
         wide_barrier();
     };
-    for (int s = 0; s < stages; s += 2) {
+    for (int s = 0; s < chunks; s += 2) {
         stage(s, 0, ring[1]);
-        if constexpr (SUB == 2) {
-            end(s);
-            if (s + 1 >= stages) break;
-        }
+        end(s);
+        if (s + 1 >= chunks) break;
         stage(s + 1, 1, ring[0]);
-        end(SUB == 2 ? s + 1 : s >> 1);
+        end(s + 1);
     }
 }
 

@@ -578,7 +578,7 @@ __device__ __forceinline__ void lin_wide_item(int b, int nb, int tiles, int ncg,
 }
 
 constexpr int LW_MB = 2;
-constexpr int LW_WAVES = 8;
+constexpr int LW_WAVES = WIDE_WAVES;
 constexpr int LW_ROWS = 16 * LW_MB * LW_WAVES;
 constexpr int LW_STRIDE = 136;                       // halves per staged output row (padded)
 
@@ -586,7 +586,7 @@ template <int K2>
 __global__ __launch_bounds__(64 * LW_WAVES) __attribute__((amdgpu_waves_per_eu(2))) void lin_wide_kernel(LinParams p)
 {
     __shared__ union {
-        WideLds<LW_WAVES> w;
+        WideLds w;
         half_t y[LW_WAVES][16 * LW_MB][LW_STRIDE];
     } lds;
     __shared__ float xs[LW_WAVES][16 * LW_MB];
@@ -606,7 +606,7 @@ __global__ __launch_bounds__(64 * LW_WAVES) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
         for (int nb = 0; nb < 8; ++nb) acc[mb][nb] = tot[mb][nb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     int range = 0, stop = nch / p.ks;                            // the chunk after the range's last
-    wide_accumulate<K2, LW_MB, LW_WAVES>(p.trellis, p.out / 16, cg, 0, nch, arow, lds.w, acc, [&](int c) {
+    wide_accumulate<K2, LW_MB>(p.trellis, p.out / 16, cg, 0, nch, arow, lds.w, acc, [&](int c) {
         if (c + 1 != stop) return;
 #pragma unroll
         for (int mb = 0; mb < LW_MB; ++mb)
@@ -752,7 +752,8 @@ size_t linear_workspace_upto(int rows, int in, int out)
     return n;
 }
 
-// Whether the decode path takes the shape: less than 2 GiB of one partial a split.
+// Whether the decode path takes the shape: its limit is 2 GiB of one partial a split and the rows. The
+// path keeps a quarter of the partials and no rows, but what it refuses stays what it is.
 bool linear_decode_fits(int rows, int in, int out)
 {
     return (size_t)linear_ksplit(rows, in, out) * rows * out * 4 + (size_t)rows * in * 2 + arrive_bytes(out) < ((size_t)1 << 31);

@@ -40,14 +40,14 @@ __device__ __forceinline__ void mfma_item_rows(const uint32_t* trellis, int nt_n
     // and the 64-row kernel's items of 1-4 row blocks since they share the GPU with the 16-row
     // kernel on another stream (512 tokens: gate/up 1319-1331 -> 1268-1287 us)
     if constexpr (MBMAX == 1) {
-        mfma_item<K2, 1, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride);
+        mfma_item<K2, 1>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride);
     } else {
         const int mb = __builtin_amdgcn_readfirstlane((rows + 15) >> 4);
         switch (mb) {
-            case 1: mfma_item<K2, 1, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
-            case 2: mfma_item<K2, 2, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
-            case 3: mfma_item<K2, 3, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
-            default: mfma_item<K2, 4, true>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+            case 1: mfma_item<K2, 1>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+            case 2: mfma_item<K2, 2>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+            case 3: mfma_item<K2, 3>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
+            default: mfma_item<K2, 4>(trellis, nt_n, cg, kt0, kt1, src, slot_of, rows, part, part_stride); break;
         }
     }
 }
