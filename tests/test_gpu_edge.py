@@ -43,6 +43,39 @@ def test_empty_rows(dev, shared):
     assert rel_err_rows(y, ref) < TOL
 
 
+@pytest.mark.parametrize("ksplit", [0, 2])
+@pytest.mark.parametrize("load,experts,shared", [
+    (17, 12, False),             # as many tiles of more than 16 rows as so many slots can have
+    (80, 6, False),              # a tile of each class an expert
+    (80, 1, True),               # the same of the shared expert (and one expert)
+    (16, 9, False),              # small tiles only, one an expert
+    (1, 40, True),               # the smallest, every slot its own; the shared expert's are one of each
+])
+def test_tile_class_bounds(dev, load, experts, shared, ksplit):
+    """Above 16 tokens the launches of a size class are sized by the most tiles it can have: routes with
+    exactly that many, by expert load. Every tile is computed (oracle)."""
+    from eva_amd import ops
+    H, I = 256, 256
+    T = load * experts
+    rng = np.random.default_rng(load + experts)
+    ex = _experts(rng, H, I, experts, 3)
+    sh = synth.expert(rng, H, I, 3, 1 / np.sqrt(H))
+    x = rng.standard_normal((T, H)).astype(np.float16)
+    sel = rng.permutation(np.repeat(np.arange(experts, dtype=np.int64), load))[:, None]
+    rw = rng.uniform(0.1, 1, size=(T, 1)).astype(np.float16)
+    ref = coop.moe_routed(x, sel, rw, ex, 10.0)
+    if shared:
+        ref = ref + coop.shared_expert(x, sh, 10.0)
+    de, ds = DeviceExperts(ex, dev), DeviceExperts([sh], dev)
+    ws = ops.MoeWorkspace(dev, rows_max=T, hidden=H, inter=I, topk=1, n_local=experts, has_shared=shared, ksplit_gu=ksplit,
+                          ksplit_down=ksplit)
+    out = torch.full((T, H), float("nan"), dtype=torch.float32, device=dev)
+    ops.moe_forward(ws, to_dev(x, dev), de.table, out, limit=10.0, bits=3, sel=to_dev(sel, dev), rw=to_dev(rw, dev),
+                    shared_ptrs=ds.ptrs(0) if shared else None, shared_bits=3 if shared else None)
+    torch.cuda.synchronize()
+    assert rel_err_rows(out.cpu().numpy(), ref) < TOL
+
+
 def test_expert_range(dev):
     from eva_amd import ops
     H, I, k, T = 256, 128, 4, 6
